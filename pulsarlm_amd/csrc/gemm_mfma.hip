@@ -566,6 +566,7 @@ __global__ void __launch_bounds__(WM * WN * 64) mfma_kernel(mfma_args a) {
                 for (int j = 0; j < NS; ++j)
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), p_rsrc,
                                                            ((i * NS + j) * NT + tid) * 16, split * TILE_BYTES, kCoherent);
+            hold_until_stored(acc);
             if (!arrive_last(&a.counters[blockIdx.x], static_cast<uint32_t>(a.splits), &last_flag)) return;
             for (int sp = 0; sp < a.splits; ++sp) {
 #pragma unroll

@@ -346,6 +346,18 @@ __device__ __forceinline__ void store_partial(float* p, float v) {
 __device__ __forceinline__ float load_partial(const float* p) {
     return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Waits for the wavefront's stores, with the accumulators live until then. A 16-byte buffer
+// store reads its data registers after it has issued; with an SGPR offset the compiler assumes
+// that a VALU write to them may follow at once, and where it reused one for the next store's
+// address (registers freed by the store) stored values were wrong while the memory pipeline
+// was busy (measured with two workgroups on a CU).
+template <int A, int B> __device__ __forceinline__ void hold_until_stored(f32x4_t (&acc)[A][B]) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int j = 0; j < B; ++j) asm volatile("" : "+v"(acc[i][j]));
+}
 // Call with every thread of the workgroup after its store_partial()s. Returns true
 // in every thread of the last workgroup to arrive at `counter`, which is then reset.
 __device__ __forceinline__ bool arrive_last(uint32_t* counter, uint32_t expected, uint32_t* lds_flag) {
