@@ -18,6 +18,10 @@ int launch_mfma(const char* op, plm_format f, const void* x, bool bf16, const vo
                 void* workspace, size_t workspace_bytes, hipStream_t s, const uint8_t* xq, const float* x_scale);
 int launch_quantize_rows(const char* op, const void* x, bool bf16, int64_t m, int64_t k, uint8_t* out, float* sx,
                          bool permuted, hipStream_t s);
+bool launch_rows(plm_format f, const void* x, bool bf16, const void* w, const void* scale, plm_dtype scale_dtype, int64_t m,
+                 int64_t n, int64_t k, int64_t block_n, int64_t group_size, void* y, void* workspace, size_t workspace_bytes,
+                 hipStream_t s);
+int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k);
 int64_t decode_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k);
 int64_t mfma_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool a8);
 
@@ -63,6 +67,26 @@ int check_gemm(const char* op, plm_format f, const void* x, plm_dtype x_dtype, c
     return PLM_OK;
 }
 
+// Checked arguments to a kernel: the rows kernel where its rule takes the call, else the decode
+// or MFMA kernels. A call is refused for its workspace by those two paths' needs alone: one
+// that is too small for the rows kernel's K split only keeps the call from it.
+int run_gemm(const char* op, plm_format f, const void* x, bool bf16, const void* w, const void* scale, plm_dtype scale_dtype,
+             int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size, void* y, void* workspace,
+             size_t workspace_bytes, hipStream_t s) {
+    const bool decode = use_decode(m, n);
+    const int64_t need = decode ? decode_workspace_bytes(f, m, n, k) : mfma_workspace_bytes(f, m, n, k, false);
+    const bool enough = need == 0 || (workspace != nullptr && static_cast<int64_t>(workspace_bytes) >= need);
+    if (enough && launch_rows(f, x, bf16, w, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace, workspace_bytes, s)) {
+        PLM_HIP_LAUNCH_CHECK(op);
+        return PLM_OK;
+    }
+    if (decode)
+        return launch_decode(op, f, x, bf16, w, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace,
+                             workspace_bytes, s, nullptr, nullptr);
+    return launch_mfma(op, f, x, bf16, w, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace, workspace_bytes, s,
+                       nullptr, nullptr);
+}
+
 }  // namespace plm
 
 using namespace plm;
@@ -71,7 +95,9 @@ extern "C" {
 
 int64_t plm_gemm_workspace_bytes(plm_format format, int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
-    return use_decode(m, n) ? decode_workspace_bytes(format, m, n, k) : mfma_workspace_bytes(format, m, n, k, false);
+    // The larger of the two paths' needs: which one a call takes also depends on its scales.
+    return std::max(rows_workspace_bytes(format, m, n, k), use_decode(m, n) ? decode_workspace_bytes(format, m, n, k)
+                                                                            : mfma_workspace_bytes(format, m, n, k, false));
 }
 
 int plm_gemm(plm_format format, const void* x, plm_dtype x_dtype, const void* weight, const void* scale,
@@ -82,12 +108,8 @@ int plm_gemm(plm_format format, const void* x, plm_dtype x_dtype, const void* we
     if (int rc = check_gemm(op, format, x, x_dtype, weight, scale, scale_dtype, m, n, k, block_n, group_size, y))
         return rc;
     if (m == 0 || n == 0) return PLM_OK;
-    const bool bf16 = x_dtype == PLM_BF16;
-    if (use_decode(m, n))
-        return launch_decode(op, format, x, bf16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y,
-                             workspace, workspace_bytes, as_stream(stream), nullptr, nullptr);
-    return launch_mfma(op, format, x, bf16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace,
-                       workspace_bytes, as_stream(stream), nullptr, nullptr);
+    return run_gemm(op, format, x, x_dtype == PLM_BF16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace,
+                    workspace_bytes, as_stream(stream));
 }
 
 }  // extern "C"
@@ -243,12 +265,8 @@ int plm_gemm_noalloc(plm_format format, const void* x, plm_dtype x_dtype, const 
     hipStream_t s = as_stream(stream);
     void* ws = nullptr;
     if (int rc = scratch_of_current_device(op, s, &ws)) return rc;
-    const bool bf16 = x_dtype == PLM_BF16;
-    if (use_decode(m, n))
-        return launch_decode(op, format, x, bf16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y, ws,
-                             static_cast<size_t>(kScratchBytes), s, nullptr, nullptr);
-    return launch_mfma(op, format, x, bf16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y, ws,
-                       static_cast<size_t>(kScratchBytes), s, nullptr, nullptr);
+    return run_gemm(op, format, x, x_dtype == PLM_BF16, weight, scale, scale_dtype, m, n, k, block_n, group_size, y, ws,
+                    static_cast<size_t>(kScratchBytes), s);
 }
 
 }  // extern "C"

@@ -1022,6 +1022,50 @@ constexpr int64_t kStageMaxM = 4;
 constexpr int64_t kStageMaxBytes = 96 * 1024;  // staging area per workgroup
 bool no_x_staging() { return knobs().decode_no_xs; }  // A/B measurements
 
+// The round-robin kernel's LDS layout for a call, and whether it takes the call.
+struct rr_layout {
+    rr_config rc;
+    int sc_mode, tpg_shift, nkt_shift, x_bytes, s_bytes, q_bytes;
+    int64_t lds;
+    bool ok;
+};
+rr_layout layout_rr(plm_format f, int64_t m, int64_t n, int64_t k, const layout_dims& d, int64_t group_size,
+                    plm_dtype scale_dtype, bool a8, bool quant_fused) {
+    rr_layout l{};
+    const int64_t tpg = group_size / kTileK;
+    l.sc_mode = d.scale_cols == 16 ? (scale_dtype == PLM_FP32 ? 1 : 0) : (scale_dtype == PLM_FP32 ? 2 : -1);
+    if (group_size % kTileK != 0 || (tpg & (tpg - 1)) != 0 || l.sc_mode < 0 || no_x_staging()) return l;
+    rr_config& rc = l.rc = choose_rr(m, n, k, f, a8 || quant_fused);
+    // The fused quantizer takes at most three tiles per wavefront: 16 wavefronts where 8
+    // would hold more (measured at N = 34816, K = 5120: 34.2 us, against 35.2 us for the
+    // separate quantizer launch and 8 wavefronts).
+    if (quant_fused && rc.sg == 1 && rc.nw == 8 && d.ktiles > 3 * 8) rc.nw = 16;
+    if (rc.sg <= 0) return l;
+    while ((int64_t{1} << l.tpg_shift) < tpg) ++l.tpg_shift;
+    const int64_t nkt = ceil_div(d.ktiles, rc.nw);
+    while ((int64_t{1} << l.nkt_shift) < nkt) ++l.nkt_shift;
+    const int64_t slots = int64_t{1} << l.nkt_shift;
+    // One batch of loads per wavefront (CH tiles) keeps every load in flight at once.
+    const int64_t ch = f == PLM_FP8 ? 4 : (rc.nw == 16 ? 2 : 4);
+    if (slots > ch) return l;
+    const int eb = l.sc_mode == 0 ? 32 : (l.sc_mode == 1 ? 64 : 4);
+    l.x_bytes = static_cast<int>(round_up(m * slots * (a8 && !quant_fused ? kTileK : 2 * kTileK), 1024));
+    // Scale copies write whole instructions: 64 lanes x (16 or 4) bytes.
+    l.s_bytes = static_cast<int>(round_up(rc.sg * slots * eb, 64 * (eb < 16 ? eb : 16)));
+    l.q_bytes = quant_fused ? static_cast<int>(round_up(m * slots * kTileK, 1024)) : 0;
+    const int64_t red = int64_t{rc.sg} * rc.nw * 64 * 16;
+    l.lds = std::max<int64_t>(int64_t{rc.nw} * (l.x_bytes + l.s_bytes + l.q_bytes) + (quant_fused ? rc.nw * 32 : 0), red);
+    // The fused quantizer's barrier needs a tile for every wavefront; its register
+    // budget holds one strip and at most three tiles per wavefront.
+    const bool fused_ok = !quant_fused || (f == PLM_FP8 && m <= 4 && rc.sg == 1 && d.ktiles >= rc.nw && d.ktiles <= 3 * rc.nw);
+    l.ok = l.lds <= 160 * 1024 && fused_ok;
+    return l;
+}
+
+bool decode_rr_takes(plm_format f, int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size, plm_dtype scale_dtype) {
+    return layout_rr(f, m, n, k, make_dims(n, k, block_n, group_size), group_size, scale_dtype, false, false).ok;
+}
+
 int launch_decode(const char* op, plm_format f, const void* x, bool bf16, const void* w, const void* scale,
                   plm_dtype scale_dtype, int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size,
                   void* y, void* workspace, size_t workspace_bytes, hipStream_t s, const uint8_t* xq,
@@ -1064,78 +1108,54 @@ int launch_decode(const char* op, plm_format f, const void* x, bool bf16, const 
         a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
     }
     const bool uniform = group_size % kTileK == 0;
-    const int64_t tpg = group_size / kTileK;
-    const int sc_mode = d.scale_cols == 16 ? (scale_dtype == PLM_FP32 ? 1 : 0) : (scale_dtype == PLM_FP32 ? 2 : -1);
-    if (uniform && (tpg & (tpg - 1)) == 0 && sc_mode >= 0 && !no_x_staging()) {
-        rr_config rc = choose_rr(m, n, k, f, xq != nullptr || quant_fused);
-        // The fused quantizer takes at most three tiles per wavefront: 16 wavefronts where 8
-        // would hold more (measured at N = 34816, K = 5120: 34.2 us, against 35.2 us for the
-        // separate quantizer launch and 8 wavefronts).
-        if (quant_fused && rc.sg == 1 && rc.nw == 8 && d.ktiles > 3 * 8) rc.nw = 16;
-        if (rc.sg > 0) {
-            rr_args r{};
-            r.x = static_cast<const uint16_t*>(x);
-            r.w = static_cast<const uint8_t*>(w);
-            r.scale = static_cast<const uint8_t*>(scale);
-            r.y = static_cast<uint16_t*>(y);
-            r.m = static_cast<int>(m);
-            r.n = static_cast<int>(n);
-            r.k = static_cast<int>(k);
-            r.ktiles = static_cast<int>(d.ktiles);
-            r.strips = static_cast<int>(d.strips);
-            r.groups = static_cast<int>(d.groups);
-            r.scale_dtype = scale_dtype;
-            r.xq = xq;
-            r.x_scale = x_scale;
-            r.quant_fused = quant_fused ? 1 : 0;
-            while ((int64_t{1} << r.tpg_shift) < tpg) ++r.tpg_shift;
-            const int64_t nkt = ceil_div(d.ktiles, rc.nw);
-            while ((int64_t{1} << r.nkt_shift) < nkt) ++r.nkt_shift;
-            const int64_t slots = int64_t{1} << r.nkt_shift;
-            const int eb = sc_mode == 0 ? 32 : (sc_mode == 1 ? 64 : 4);
-            r.x_bytes = static_cast<int>(round_up(m * slots * (xq != nullptr ? kTileK : 2 * kTileK), 1024));
-            // Scale copies write whole instructions: 64 lanes x (16 or 4) bytes.
-            const int64_t cs = eb < 16 ? eb : 16;
-            const int64_t s_bytes = round_up(rc.sg * slots * eb, 64 * cs);
-            // Fused quantizer: the wavefront's e4m3 x after its scales; after every wavefront's
-            // area, the row maxima of all wavefronts, then their row scales (4 rows x fp32).
-            r.qx_off = static_cast<int>(r.x_bytes + s_bytes);
-            const int64_t q_bytes = quant_fused ? round_up(m * slots * kTileK, 1024) : 0;
-            r.wave_bytes = static_cast<int>(r.x_bytes + s_bytes + q_bytes);
-            r.amax_off = rc.nw * r.wave_bytes;
-            const int64_t red = int64_t{rc.sg} * rc.nw * 64 * 16;
-            const int64_t lds = std::max<int64_t>(int64_t{rc.nw} * r.wave_bytes + (quant_fused ? rc.nw * 32 : 0), red);
-            // One batch of loads per wavefront (CH tiles) keeps every load in flight at once.
-            const int64_t ch = f == PLM_FP8 ? 4 : (rc.nw == 16 ? 2 : 4);
-            // The fused quantizer's barrier needs a tile for every wavefront; its register
-            // budget holds one strip and at most three tiles per wavefront.
-            const bool fused_ok = !quant_fused || (f == PLM_FP8 && m <= 4 && rc.sg == 1 && d.ktiles >= rc.nw &&
-                                                   d.ktiles <= 3 * rc.nw);
-            if (lds <= 160 * 1024 && slots <= ch && fused_ok) {
-                const size_t l = static_cast<size_t>(lds);
-                // CH: tiles per load batch (all of a wavefront's tiles at K = 4096).
-                if (f == PLM_INT4) {
-                    if (rc.nw == 16) {
-                        if (bf16) launch_rr_sg<PLM_INT4, true, 16, 2>(r, sc_mode, rc.sg, l, s);
-                        else launch_rr_sg<PLM_INT4, false, 16, 2>(r, sc_mode, rc.sg, l, s);
-                    } else {
-                        if (bf16) launch_rr_sg<PLM_INT4, true, 8, 4>(r, sc_mode, rc.sg, l, s);
-                        else launch_rr_sg<PLM_INT4, false, 8, 4>(r, sc_mode, rc.sg, l, s);
-                    }
-                } else {
-                    // fp8 (K = 5120 at the Qwen3-27B shapes: 40 tiles, up to 3 per wavefront).
-                    if (rc.nw == 16) {
-                        if (bf16) launch_rr_sg<PLM_FP8, true, 16, 4>(r, sc_mode, rc.sg, l, s);
-                        else launch_rr_sg<PLM_FP8, false, 16, 4>(r, sc_mode, rc.sg, l, s);
-                    } else {
-                        if (bf16) launch_rr_sg<PLM_FP8, true, 8, 4>(r, sc_mode, rc.sg, l, s);
-                        else launch_rr_sg<PLM_FP8, false, 8, 4>(r, sc_mode, rc.sg, l, s);
-                    }
-                }
-                PLM_HIP_LAUNCH_CHECK(op);
-                return PLM_OK;
+    const rr_layout l = layout_rr(f, m, n, k, d, group_size, scale_dtype, xq != nullptr, quant_fused);
+    if (l.ok) {
+        const rr_config& rc = l.rc;
+        rr_args r{};
+        r.x = static_cast<const uint16_t*>(x);
+        r.w = static_cast<const uint8_t*>(w);
+        r.scale = static_cast<const uint8_t*>(scale);
+        r.y = static_cast<uint16_t*>(y);
+        r.m = static_cast<int>(m);
+        r.n = static_cast<int>(n);
+        r.k = static_cast<int>(k);
+        r.ktiles = static_cast<int>(d.ktiles);
+        r.strips = static_cast<int>(d.strips);
+        r.groups = static_cast<int>(d.groups);
+        r.scale_dtype = scale_dtype;
+        r.xq = xq;
+        r.x_scale = x_scale;
+        r.quant_fused = quant_fused ? 1 : 0;
+        r.tpg_shift = l.tpg_shift;
+        r.nkt_shift = l.nkt_shift;
+        r.x_bytes = l.x_bytes;
+        // Fused quantizer: the wavefront's e4m3 x after its scales; after every wavefront's
+        // area, the row maxima of all wavefronts, then their row scales (4 rows x fp32).
+        r.qx_off = l.x_bytes + l.s_bytes;
+        r.wave_bytes = l.x_bytes + l.s_bytes + l.q_bytes;
+        r.amax_off = rc.nw * r.wave_bytes;
+        const size_t lds = static_cast<size_t>(l.lds);
+        // CH: tiles per load batch (all of a wavefront's tiles at K = 4096; fp8 at the Qwen3-27B
+        // shapes, K = 5120: 40 tiles, up to 3 per wavefront).
+        if (f == PLM_INT4) {
+            if (rc.nw == 16) {
+                if (bf16) launch_rr_sg<PLM_INT4, true, 16, 2>(r, l.sc_mode, rc.sg, lds, s);
+                else launch_rr_sg<PLM_INT4, false, 16, 2>(r, l.sc_mode, rc.sg, lds, s);
+            } else {
+                if (bf16) launch_rr_sg<PLM_INT4, true, 8, 4>(r, l.sc_mode, rc.sg, lds, s);
+                else launch_rr_sg<PLM_INT4, false, 8, 4>(r, l.sc_mode, rc.sg, lds, s);
+            }
+        } else {
+            if (rc.nw == 16) {
+                if (bf16) launch_rr_sg<PLM_FP8, true, 16, 4>(r, l.sc_mode, rc.sg, lds, s);
+                else launch_rr_sg<PLM_FP8, false, 16, 4>(r, l.sc_mode, rc.sg, lds, s);
+            } else {
+                if (bf16) launch_rr_sg<PLM_FP8, true, 8, 4>(r, l.sc_mode, rc.sg, lds, s);
+                else launch_rr_sg<PLM_FP8, false, 8, 4>(r, l.sc_mode, rc.sg, lds, s);
             }
         }
+        PLM_HIP_LAUNCH_CHECK(op);
+        return PLM_OK;
     }
     if (quant_fused) {
         // The split-K kernel with the quantizer fused: one workgroup over all of K (the row

@@ -412,6 +412,9 @@ struct tuning {
     int decode_sp = 0, decode_tpw = 0, decode_nw = 0;  // PLM_DECODE="sp,tpw,nw"
     int rr_sg = -1, rr_nw = 0;         // PLM_DECODE_RR="sg,nw" (sg 0: round-robin kernel off)
     bool decode_no_xs = false;         // PLM_DECODE_NO_XS: x from global memory, not LDS
+    bool rows_off = false;             // PLM_ROWS=0: no rows kernel
+    bool rows_force = false;           // PLM_ROWS=1 or a shape: wherever it can
+    int rows_sg = 0, rows_splits = 0;  // PLM_ROWS="sg,splits": its strips per workgroup and K splits
     char mfma_shape = 0;               // PLM_MFMA=<letter>: force one MFMA tile shape
     bool mfma_no_halves = false;       // PLM_MFMA_NO_HALVES
     bool mfma_no_tail = false;         // PLM_MFMA_NO_TAIL

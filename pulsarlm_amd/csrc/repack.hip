@@ -64,6 +64,13 @@ tuning parse_tuning() {
             t.rr_sg = sg, t.rr_nw = nw;
     }
     t.decode_no_xs = env("PLM_DECODE_NO_XS") != nullptr;
+    if (const char* e = env("PLM_ROWS")) {
+        int sg = 0, splits = 0;
+        const int got = sscanf(e, "%d,%d", &sg, &splits);
+        t.rows_off = got >= 1 && sg == 0;
+        t.rows_force = got >= 1 && sg > 0;
+        if (got == 2 && sg >= 1 && sg <= 4 && splits >= 1 && splits <= 8) t.rows_sg = sg, t.rows_splits = splits;
+    }
     if (const char* e = env("PLM_MFMA")) t.mfma_shape = e[0];
     t.mfma_no_halves = env("PLM_MFMA_NO_HALVES") != nullptr;
     t.mfma_no_tail = env("PLM_MFMA_NO_TAIL") != nullptr;
