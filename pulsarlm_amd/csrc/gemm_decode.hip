@@ -67,20 +67,6 @@ __device__ __forceinline__ float div_by_scale(float x, float s, float inv) {
     return copysignf(__builtin_fmaf(__builtin_fmaf(-q, s, x), inv, q), x);
 }
 
-template <int CTRL, int ROW_MASK> __device__ __forceinline__ float dpp_f32(float x) {
-    const int i = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, ROW_MASK, 0xf, false));
-}
-__device__ __forceinline__ float wave_max_to_lane63(float v) {
-    v = fmaxf(v, dpp_f32<0xB1, 0xf>(v));   // quad_perm [1,0,3,2]
-    v = fmaxf(v, dpp_f32<0x4E, 0xf>(v));   // quad_perm [2,3,0,1]
-    v = fmaxf(v, dpp_f32<0x141, 0xf>(v));  // row_half_mirror
-    v = fmaxf(v, dpp_f32<0x140, 0xf>(v));  // row_mirror
-    v = fmaxf(v, dpp_f32<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
-    v = fmaxf(v, dpp_f32<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
 // One wavefront's batch of TPW K tiles for SP strips: weights, raw scale bits and x (RB
 // blocks of 16 rows).
 template <plm_format F, int SP, int TPW, bool A8, int RB> struct decode_batch {

@@ -374,6 +374,40 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, uint32_t expected
 }
 
 // ---------------------------------------------------------------------------
+// Wavefront reductions and scans by DPP: within each row of 16 lanes, then the row broadcasts
+// carry row 0 into row 1 and rows 0-1 into rows 2-3. No LDS round trips (a ds_bpermute shuffle
+// is one each).
+// ---------------------------------------------------------------------------
+template <int CTRL, int ROW_MASK> __device__ __forceinline__ float dpp_f32(float x) {
+    const int i = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ float wave_max_to_lane63(float v) {
+    v = fmaxf(v, dpp_f32<0xB1, 0xf>(v));   // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp_f32<0x4E, 0xf>(v));   // quad_perm [2,3,0,1]
+    v = fmaxf(v, dpp_f32<0x141, 0xf>(v));  // row_half_mirror
+    v = fmaxf(v, dpp_f32<0x140, 0xf>(v));  // row_mirror
+    v = fmaxf(v, dpp_f32<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
+    v = fmaxf(v, dpp_f32<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wave_max_to_lane63(v)), 63));
+}
+template <int CTRL, int ROW_MASK> __device__ __forceinline__ int dpp_add(int x) {
+    return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROW_MASK, 0xf, true);
+}
+// Inclusive prefix sum over the wavefront.
+__device__ __forceinline__ int wave_inclusive_scan(int x) {
+    x = dpp_add<0x111, 0xf>(x);  // row_shr:1
+    x = dpp_add<0x112, 0xf>(x);  // row_shr:2
+    x = dpp_add<0x114, 0xf>(x);  // row_shr:4
+    x = dpp_add<0x118, 0xf>(x);  // row_shr:8
+    x = dpp_add<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+}
+
+// ---------------------------------------------------------------------------
 // Host-side error plumbing.
 // ---------------------------------------------------------------------------
 void set_error(const char* op, const char* fmt, ...);

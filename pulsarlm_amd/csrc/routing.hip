@@ -96,6 +96,97 @@ __global__ void __launch_bounds__(kRouteWaves * 64)
     }
 }
 
+// The same for up to 64 EPL experts with the probabilities in registers (lane l holds experts l,
+// l + 64, ..): each round's maximum is a DPP reduction, the winner's expert comes from the one lane
+// that holds it (the lowest expert where several do), with no LDS round trips, which were the time
+// of the kernel above: k rounds of six shuffles of two values. k = 8, the kernel above and this one:
+// 8 tokens 8.0 and 4.0 us with 128 experts, 15.2 and 5.9 with 512, 24.1 and 9.3 with 1024; 4096
+// tokens 9.7 and 5.8, 17.0 and 9.3, 27.7 and 15.3. Above 1024 experts (16 probabilities a lane) no
+// model of the framework goes, and the LDS kernel takes them. Same results bit for bit: the sum
+// keeps its butterfly.
+template <int DT, int EPL>
+__global__ void __launch_bounds__(kRouteWaves * 64)
+    route_top_k_reg_kernel(const void* logits, int64_t row_stride, int64_t tokens, int experts, int k, float* weights,
+                           int64_t* chosen64, int32_t* chosen32) {
+    const int lane = threadIdx.x & 63;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * kRouteWaves + (threadIdx.x >> 6);
+    if (t >= tokens) return;  // wave-uniform; nothing below synchronizes the workgroup
+    const int64_t base = t * row_stride;
+    float q[EPL];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+        const int e = lane + 64 * i;
+        q[i] = e < experts ? value_at<DT>(logits, base + e) : -INFINITY;
+        mx = fmaxf(mx, q[i]);
+    }
+    mx = wave_max(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+        if (lane + 64 * i >= experts) continue;
+        q[i] = expf(q[i] - mx);
+        sum += q[i];
+    }
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    float bv = -INFINITY;  // this lane's best remaining probability and its expert
+    int be = experts;
+    auto rescan = [&]() {
+        bv = -INFINITY;
+        be = experts;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i)
+            if (q[i] > bv) bv = q[i], be = lane + 64 * i;  // the lower expert first among equals
+    };
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) q[i] = lane + 64 * i < experts ? q[i] / sum : -INFINITY;
+    rescan();
+
+    float my_top = 0.f;
+    int my_expert = 0;
+    for (int j = 0; j < k; ++j) {
+        // `experts` and -inf where nothing is left to rank (NaN probabilities).
+        const float v = wave_max(bv);
+        uint64_t tied = __ballot(bv == v);
+        int e = experts;
+        while (tied != 0) {  // wave-uniform; one pass unless probabilities are equal
+            const int l = __builtin_ctzll(tied);
+            e = min(e, __builtin_amdgcn_readlane(be, l));
+            tied &= tied - 1;
+        }
+        if (lane == j) my_top = v, my_expert = e;
+        if (be == e && e < experts) {  // the owner drops the winner and finds its next best
+#pragma unroll
+            for (int i = 0; i < EPL; ++i)
+                if (lane + 64 * i == e) q[i] = -INFINITY;
+            rescan();
+        }
+    }
+    float total = 0.f;
+    for (int j = 0; j < k; ++j)
+        total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_top), j));
+    if (lane < k) {
+        weights[t * k + lane] = my_top / total;
+        if (chosen64 != nullptr) chosen64[t * k + lane] = my_expert;
+        if (chosen32 != nullptr) chosen32[t * k + lane] = my_expert;
+    }
+}
+
+template <int DT>
+void launch_route(const void* logits, int64_t row_stride, int64_t tokens, int experts, int k, float* weights,
+                  int64_t* chosen64, int32_t* chosen32, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(tokens, kRouteWaves)));
+    constexpr int threads = kRouteWaves * 64;
+    if (experts <= 64) route_top_k_reg_kernel<DT, 1><<<grid, threads, 0, s>>>(logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+    else if (experts <= 128) route_top_k_reg_kernel<DT, 2><<<grid, threads, 0, s>>>(logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+    else if (experts <= 256) route_top_k_reg_kernel<DT, 4><<<grid, threads, 0, s>>>(logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+    else if (experts <= 512) route_top_k_reg_kernel<DT, 8><<<grid, threads, 0, s>>>(logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+    else if (experts <= 1024) route_top_k_reg_kernel<DT, 16><<<grid, threads, 0, s>>>(logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+    else
+        route_top_k_kernel<DT><<<grid, threads, static_cast<size_t>(kRouteWaves) * experts * sizeof(float), s>>>(
+            logits, row_stride, tokens, experts, k, weights, chosen64, chosen32);
+}
+
 template <int DT> __device__ __forceinline__ float round_dt(float v) {
     if constexpr (DT == PLM_FP32) return v;
     else return round_to<DT == PLM_BF16>(v);
@@ -172,15 +263,10 @@ int plm_route_top_k(const void* logits, plm_dtype dtype, int64_t tokens, int64_t
     PLM_CHECK_ARG(logits != nullptr && weights != nullptr && (chosen != nullptr || chosen_i32 != nullptr), op,
                   "null pointer");
     const hipStream_t s = as_stream(stream);
-    const dim3 grid(static_cast<unsigned>(ceil_div(tokens, kRouteWaves)));
-    const size_t lds = static_cast<size_t>(kRouteWaves) * experts * sizeof(float);
     const int e = static_cast<int>(experts), kk = static_cast<int>(k);
-    if (dtype == PLM_FP32)
-        route_top_k_kernel<PLM_FP32><<<grid, kRouteWaves * 64, lds, s>>>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32);
-    else if (dtype == PLM_BF16)
-        route_top_k_kernel<PLM_BF16><<<grid, kRouteWaves * 64, lds, s>>>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32);
-    else
-        route_top_k_kernel<PLM_FP16><<<grid, kRouteWaves * 64, lds, s>>>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32);
+    if (dtype == PLM_FP32) launch_route<PLM_FP32>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32, s);
+    else if (dtype == PLM_BF16) launch_route<PLM_BF16>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32, s);
+    else launch_route<PLM_FP16>(logits, row_stride, tokens, e, kk, weights, chosen, chosen_i32, s);
     PLM_HIP_LAUNCH_CHECK(op);
     return PLM_OK;
 }
