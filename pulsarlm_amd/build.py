@@ -22,8 +22,8 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libpulsarlm_amd.so"
 
-SOURCES = ["repack.hip", "gemm_decode.hip", "gemm_mfma.hip", "gemm_rows_int4.hip", "gemm_rows_fp8.hip",
-           "quant.hip", "moe.hip", "routing.hip", "gemm_plain.hip", "capi.hip"]
+SOURCES = ["repack.hip", "gemm_decode.hip", "gemm_mfma.hip", "gemm_mfma_int4.hip", "gemm_mfma_fp8.hip", "gemm_mfma_a8.hip",
+           "gemm_mfma_grouped.hip", "gemm_rows_int4.hip", "gemm_rows_fp8.hip", "quant.hip", "moe.hip", "routing.hip", "gemm_plain.hip", "capi.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -44,7 +44,7 @@ FLAGS = [
 # v_mfma): with the default AGPR form the register allocator splits the accumulator set
 # between the two files and copies it back and forth every K step.
 SOURCE_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-                for src in ("gemm_mfma.hip", "gemm_rows_int4.hip", "gemm_rows_fp8.hip")}
+                for src in SOURCES if src.startswith(("gemm_mfma", "gemm_rows"))}
 
 
 EXTRA_DEFINES: list[str] = []

@@ -24,6 +24,7 @@ bool launch_rows(plm_format f, const void* x, bool bf16, const void* w, const vo
 int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k);
 int64_t decode_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k);
 int64_t mfma_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool a8);
+int64_t mfma_contract(plm_format f, int64_t m, int64_t n, int64_t k, bool a8);
 
 // Decode kernels or MFMA kernel. The decode kernels take up to 32 rows (one or two 16-row
 // MFMA blocks; W8A8 one). Measured on MI355X at the Qwen3-8B shapes (both paths at every M
@@ -74,7 +75,7 @@ int run_gemm(const char* op, plm_format f, const void* x, bool bf16, const void*
              int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size, void* y, void* workspace,
              size_t workspace_bytes, hipStream_t s) {
     const bool decode = use_decode(m, n);
-    const int64_t need = decode ? decode_workspace_bytes(f, m, n, k) : mfma_workspace_bytes(f, m, n, k, false);
+    const int64_t need = decode ? decode_workspace_bytes(f, m, n, k) : mfma_contract(f, m, n, k, false);
     const bool enough = need == 0 || (workspace != nullptr && static_cast<int64_t>(workspace_bytes) >= need);
     if (enough && launch_rows(f, x, bf16, w, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace, workspace_bytes, s)) {
         PLM_HIP_LAUNCH_CHECK(op);
@@ -120,15 +121,17 @@ namespace {
 struct w8a8_ws {
     int64_t gemm, xq, sx, total;
 };
-w8a8_ws w8a8_layout(int64_t m, int64_t n, int64_t k) {
+// The GEMM region holds its plan's partial sums where `have` bytes allow it, else what every call brings.
+w8a8_ws w8a8_layout(int64_t m, int64_t n, int64_t k, int64_t have) {
     w8a8_ws w{};
-    // The split-K counters always keep the front of the workspace, even when this call
-    // does not split, so scratch written here never lands on them.
-    const int64_t gemm = use_decode_w8a8(m) ? decode_workspace_bytes(PLM_FP8, m, n, k)
-                                            : mfma_workspace_bytes(PLM_FP8, m, n, k, true);
-    w.gemm = round_up(std::max<int64_t>(gemm, kCounterBytes), 256);
     w.xq = round_up(m * ceil_div(k, kTileK) * kTileK, 256);
     w.sx = round_up(m * 4, 256);
+    // The split-K counters always keep the front of the workspace, even when this call
+    // does not split, so scratch written here never lands on them.
+    auto region = [&](int64_t gemm) { return round_up(std::max<int64_t>(gemm, kCounterBytes), 256); };
+    const bool decode = use_decode_w8a8(m);
+    w.gemm = region(decode ? decode_workspace_bytes(PLM_FP8, m, n, k) : mfma_workspace_bytes(PLM_FP8, m, n, k, true));
+    if (!decode && w.gemm + w.xq + w.sx > have) w.gemm = region(mfma_contract(PLM_FP8, m, n, k, true));
     w.total = w.gemm + w.xq + w.sx;
     return w;
 }
@@ -151,7 +154,7 @@ int plm_quantize_rows_e4m3(const void* x, plm_dtype x_dtype, int64_t m, int64_t 
 
 int64_t plm_gemm_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
-    return w8a8_layout(m, n, k).total;
+    return w8a8_layout(m, n, k, INT64_MAX).total;
 }
 
 int plm_gemm_w8a8(const void* x, plm_dtype x_dtype, const void* weight, const void* scale, plm_dtype scale_dtype,
@@ -163,7 +166,7 @@ int plm_gemm_w8a8(const void* x, plm_dtype x_dtype, const void* weight, const vo
         return rc;
     PLM_CHECK_ARG(group_size % kTileK == 0, op, "group_size must be a multiple of 128 for the fp8 MFMA");
     if (m == 0 || n == 0) return PLM_OK;
-    const w8a8_ws l = w8a8_layout(m, n, k);
+    const w8a8_ws l = w8a8_layout(m, n, k, workspace != nullptr ? static_cast<int64_t>(workspace_bytes) : 0);
     if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < l.total) {
         set_error(op, "workspace of %lld bytes required, %zu given", static_cast<long long>(l.total), workspace_bytes);
         return PLM_ERR_WORKSPACE;

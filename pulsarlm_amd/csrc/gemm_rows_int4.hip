@@ -82,9 +82,8 @@ struct rows_cost {
 constexpr rows_cost kRowsInt4{0.0332, {0.0414, 0.0464, 0.0641, 0.0697}, 0.864, 0.812, 0.286, 0.161, 0.279};
 constexpr rows_cost kRowsFp8{0.0402, {0.0641, 0.0692, 0.0847, 0.0855}, 0.873, 0.871, 0.412, 0.180, 0.281};
 
-rows_plan plan_rows(plm_format f, int64_t m, int64_t n, int64_t k) {
+rows_plan make_rows_plan(plm_format f, int64_t m, int64_t n, int64_t k) {
     rows_plan best;
-    if (m < 1 || m > kRowsMaxM || k > kRowsMaxK || n > (int64_t{1} << 24)) return best;
     const int64_t strips = ceil_div(n, kTileN), ktiles = ceil_div(k, kTileK), cus = cu_count();
     if (strips * ktiles * tile_bytes(f) >= kOOB) return best;
     const int64_t m_blocks = ceil_div(m, 64);  // above 64 rows: two row blocks
@@ -119,23 +118,28 @@ rows_plan plan_rows(plm_format f, int64_t m, int64_t n, int64_t k) {
     return best;
 }
 
+rows_plan plan_rows(plm_format f, int64_t m, int64_t n, int64_t k) {
+    if (m < 1 || m > kRowsMaxM || k > kRowsMaxK || n > (int64_t{1} << 24)) return rows_plan{};
+    thread_local plan_cache<rows_plan> cache;
+    return cache.get(f, m, n, k, [&] { return make_rows_plan(f, m, n, k); });
+}
+
 static int64_t rows_need(const rows_plan& p) {
     if (p.rb == 0 || p.splits <= 1) return 0;
     return kCounterBytes + static_cast<int64_t>(p.m_blocks) * p.n_blocks * p.splits * p.rb * p.sg * 1024;
 }
 int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k) { return rows_need(plan_rows(f, m, n, k)); }
 
-// The rows kernel or the decode / MFMA kernels, by both sides' times at the layers above and
-// at 22 random ones (hidden 2048..5120, M = 1..112; us, without -> with the rows kernel). rr: the
+// The rows kernel or the decode / MFMA kernels, by both sides' times at the layers above and at 31
+// random ones (hidden 2048..5120, M = 1..128; us, without -> with the rows kernel). rr: the
 // round-robin decode kernel takes the call.
-// * 17 to 64 rows: the rows kernel (int4 1.03-1.9x, fp8 1.1-2.1x), but int4 above 48 rows with
-//   four strips or more per CU (K 2816, N 16896, M = 64: 20.6 -> 21.8; K 4096, N 24576: 28.0 -> 27.3) and
-//   above 32 with four to five (K 3584, N 16896, M = 48: 23.4 -> 25.3; K 4096, N 24576: 27.3 -> 24.2).
-// * Above 64 the weights are read once per row block: its lead is gone where the tiles make
-//   many rounds. int4 up to 96 rows at any width (K 4096, N 24576: 47.2 -> 40.4) and to 128 up to two
-//   strips per CU (N 6144: 19.7 -> 14.4; K 2944, N 11776, M = 112: 21.6 -> 22.7); fp8 up to six (K 3840,
-//   N 20992, M = 80: 68.3 -> 47.3; K 5120, N 34816, M = 96: 88 -> 98); groups below 128 always (K 4096,
-//   N 24576, g32, M = 100: 57.9 -> 48.6).
+// * 17 to 64 rows: the rows kernel (against the MFMA kernel int4 1.1-2.0x, fp8 1.01-1.8x), but int4
+//   above 32 rows with more than four strips per CU, where the MFMA kernel is even or faster (K 4736,
+//   N 21248, M = 64: 28.6 -> 32.7) unless three-strip tiles nearly fill whole rounds of the CUs and there
+//   are at most 48 rows (K 5120, N 23040: M = 36 31.0 -> 29.3, M = 48 30.5 -> 30.7).
+// * Above 64 the weights are read once per row block: up to two strips per CU and K = 8448 (int4
+//   K 4736, N 5248, M = 96: 19.4 -> 15.0, K 8192, N 2432, M = 128: 16.2 -> 15.4; fp8 K 2944, N 3968, M = 128:
+//   18.8 -> 11.0; beyond: int4 K 2048, N 8704, M = 96 14.3 -> 15.2, K 9088, N 3200, M = 112 21.8 -> 24.8).
 // * Up to 16 rows int4: the round-robin kernel where it applies (3-8 % faster), but above 4 rows
 //   with five strips or more per CU (K 4096, N 24576, M = 16: 15.4 -> 14.6). Elsewhere (long K,
 //   groups below 128) the rows kernel (K 14336, N 5120, M = 1: 14.9 -> 12.3; K 8192, N 8192: 12.3 -> 9.6), but
@@ -153,8 +157,11 @@ bool use_rows(plm_format f, int64_t m, int64_t n, int64_t k, int64_t group_size,
     if (t.rows_off || t.decode_max_m >= 0 || t.decode_sp > 0 || t.rr_sg > 0 || t.decode_no_xs || t.mfma_shape) return false;
     const int64_t strips = ceil_div(n, kTileN), cus = cu_count();
     const bool sub = group_size % kTileK != 0;
-    if (m > 64) return sub || (f == PLM_FP8 ? strips <= 6 * cus : m <= 96 || strips <= 2 * cus);
-    if (m > 16) return f == PLM_FP8 || sub || strips < 4 * cus || m <= (strips < 5 * cus ? 32 : 48);
+    if (m > 64) return strips <= 2 * cus && k <= 66 * kTileK;
+    if (m > 16) {
+        const int64_t tiles3 = ceil_div(strips, 3);
+        return f == PLM_FP8 || m <= 32 || strips <= 4 * cus || (m <= 48 && 10 * tiles3 >= 9 * round_up(tiles3, cus));
+    }
     if (f == PLM_FP8) {
         if (strips >= 4 * cus && m <= (rr ? 4 : 2)) return false;
         if (strips <= cus) return m <= 4 ? rr || m > 2 : !(rr || k <= 5120);

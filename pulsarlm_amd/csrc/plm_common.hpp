@@ -449,7 +449,8 @@ struct tuning {
     bool rows_off = false;             // PLM_ROWS=0: no rows kernel
     bool rows_force = false;           // PLM_ROWS=1 or a shape: wherever it can
     int rows_sg = 0, rows_splits = 0;  // PLM_ROWS="sg,splits": its strips per workgroup and K splits
-    char mfma_shape = 0;               // PLM_MFMA=<letter>: force one MFMA tile shape
+    char mfma_shape = 0;               // PLM_MFMA=<letter>[,splits]: force one MFMA tile shape (and K split)
+    int mfma_splits = 0;
     bool mfma_no_halves = false;       // PLM_MFMA_NO_HALVES
     bool mfma_no_tail = false;         // PLM_MFMA_NO_TAIL
     bool mfma_unsplit = false;         // PLM_MFMA_UNSPLIT: no K split and no tail launch
@@ -457,7 +458,31 @@ struct tuning {
     bool moe_small_sort_off = false;   // PLM_MOE_SMALL_SORT=0
     bool moe_unfused = false;          // PLM_MOE_UNFUSED
     bool moe_persist = false;          // PLM_MOE_PERSIST=1: persistent grouped launches
+    unsigned epoch = 0;                // one more with each re-parse
 };
 const tuning& knobs();
+
+// The plans of the last sizes a thread has called with (a pure function of the sizes and the
+// knobs; working one out takes a few us, as long as a short kernel): 64 entries per thread.
+template <typename P> struct plan_cache {
+    struct entry {
+        int64_t m = -1, n = 0, k = 0;
+        int kind = 0;
+        unsigned epoch = 0;
+        P plan{};
+    };
+    entry entries[64];
+    template <typename Fn> const P& get(int kind, int64_t m, int64_t n, int64_t k, Fn make) {
+        const uint64_t h = (static_cast<uint64_t>(m) * 0x9E3779B97F4A7C15u) ^ (static_cast<uint64_t>(n) * 0xC2B2AE3D27D4EB4Fu) ^
+                           (static_cast<uint64_t>(k) * 0x165667B19E3779F9u) ^ static_cast<uint64_t>(kind);
+        entry& e = entries[(h ^ (h >> 29)) >> 7 & 63];
+        const unsigned epoch = knobs().epoch;
+        if (e.m != m || e.n != n || e.k != k || e.kind != kind || e.epoch != epoch) {
+            e.plan = make();
+            e.m = m, e.n = n, e.k = k, e.kind = kind, e.epoch = epoch;
+        }
+        return e.plan;
+    }
+};
 
 }  // namespace plm

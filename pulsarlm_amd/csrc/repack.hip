@@ -71,7 +71,10 @@ tuning parse_tuning() {
         t.rows_force = got >= 1 && sg > 0;
         if (got == 2 && sg >= 1 && sg <= 4 && splits >= 1 && splits <= 8) t.rows_sg = sg, t.rows_splits = splits;
     }
-    if (const char* e = env("PLM_MFMA")) t.mfma_shape = e[0];
+    if (const char* e = env("PLM_MFMA")) {
+        t.mfma_shape = e[0];
+        if (e[0] != 0 && e[1] == ',') t.mfma_splits = atoi(e + 2);
+    }
     t.mfma_no_halves = env("PLM_MFMA_NO_HALVES") != nullptr;
     t.mfma_no_tail = env("PLM_MFMA_NO_TAIL") != nullptr;
     t.mfma_unsplit = env("PLM_MFMA_UNSPLIT") != nullptr;
@@ -395,7 +398,9 @@ extern "C" {
 // thread-safe against concurrent GEMM calls.
 __attribute__((visibility("default"))) void plm_internal_reload_tuning() {
     std::lock_guard<std::mutex> lock(plm::g_tuning_mutex);
+    const unsigned epoch = plm::g_tuning.epoch + 1;
     plm::g_tuning = plm::parse_tuning();
+    plm::g_tuning.epoch = epoch;
     plm::g_tuning_parsed = true;
 }
 }  // extern "C"

@@ -1,0 +1,85 @@
+"""Every tile shape and K split of the MFMA kernel, at row counts around its tile edges, against the
+dequantized weights (pinned to the oracle elsewhere) in float64."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from pulsarlm_amd import ops
+from tests._util import TDT, assert_close, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
+
+pytestmark = pytest.mark.gpu
+
+# N = 1016: the last strip is half empty and no shape's strips divide its 64; K = 1152: 9 K tiles.
+N, K = 1016, 1152
+ROWS = {"R": 64, "W": 256, "X": 256, "Q": 64, "H": 128, "B": 128, "C": 96, "D": 112, "F": 96, "A": 128, "G": 256, "S": 128}
+
+
+@pytest.fixture(autouse=True)
+def no_rows_kernel(tuning_env):
+    tuning_env("PLM_ROWS", "0")
+
+
+@pytest.mark.parametrize("g,dtype,sdt", [(128, "bf16", "fp16"), (32, "fp16", "fp16"), (48, "bf16", "fp32"), (384, "bf16", "fp32")])
+@pytest.mark.parametrize("shape", list("RWXQHBCDF"))
+def test_int4_shapes(shape, g, dtype, sdt, tuning_env):
+    packed, s = int4_case(N, K, g, 1, seed=g)
+    s = s.astype(np.float16 if sdt == "fp16" else np.float32)
+    w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), scale_tensor(s), 1, g)
+    dense = ops.dequant_marlin_cuda("int4", w, sc, N, K, 1, g, TDT[dtype]).double()
+    for m in (33, ROWS[shape] - 1, ROWS[shape] + 1, 3 * ROWS[shape] + 17):
+        x = to_dev(x_case(m, K, dtype, seed=m), TDT[dtype])
+        ref = to_np(x.double() @ dense.t())
+        for splits in (1, 3, 8):
+            tuning_env("PLM_MFMA", f"{shape},{splits}")
+            y = ops.gemm_int4_marlin_cuda(x, w, sc, N, 1, g)
+            assert_close(y, ref, f"{shape} m={m} splits={splits}")
+            assert torch.equal(y, ops.gemm_int4_marlin_cuda(x, w, sc, N, 1, g)), "not deterministic"
+
+
+@pytest.mark.parametrize("block_n,dtype", [(128, "bf16"), (1, "fp16")])
+@pytest.mark.parametrize("shape", list("RXGABCDF"))
+def test_fp8_shapes(shape, block_n, dtype, tuning_env):
+    codes, s = fp8_case(N, K, 128, block_n, seed=5)
+    w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), scale_tensor(s), block_n, 128)
+    dense = ops.dequant_marlin_cuda("fp8", w, sc, N, K, block_n, 128, TDT[dtype]).double()
+    for m in (33, ROWS[shape] - 1, ROWS[shape] + 1, 2 * ROWS[shape] + 17):
+        x = to_dev(O.round_to(x_case(m, K, dtype, seed=m) * np.float32(0.05), dtype), TDT[dtype])
+        ref = to_np(x.double() @ dense.t())
+        for splits in (1, 3, 8):
+            tuning_env("PLM_MFMA", f"{shape},{splits}")
+            assert_close(ops.gemm_fp8_marlin_cuda(x, w, sc, N, block_n, 128), ref, f"{shape} m={m} splits={splits}")
+
+
+@pytest.mark.parametrize("shape", list("SRWXHABCD"))
+def test_w8a8_shapes(shape, tuning_env):
+    rng = np.random.default_rng(7)
+    codes, scale = O.fp8_block_quantize(O.bf16_round(rng.standard_normal((N, K)).astype(np.float32) * 0.02), 128, 128)
+    w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), to_dev(scale), 128, 128)
+    for m in (33, ROWS[shape] - 1, ROWS[shape] + 1, 2 * ROWS[shape] + 17):
+        x = x_case(m, K, "bf16", seed=m)
+        xc, xs = O.quantize_per_token_e4m3(x)
+        ref = O.gemm_w8a8_ref(xc, xs, codes, scale, 128, 128, dtype=None)
+        for splits in (1, 3, 8):
+            tuning_env("PLM_MFMA", f"{shape},{splits}")
+            y = ops.gemm_fp8_w8a8_cuda(to_dev(x, torch.bfloat16), w, sc, N, 128, 128)
+            assert_close(y, ref, f"{shape} m={m} splits={splits}")
+
+
+def test_random_sizes_by_the_rule(tuning_env):
+    """The plan's own pick at random sizes, ragged in every dimension."""
+    tuning_env("PLM_ROWS", None)
+    rng = np.random.default_rng(3)
+    for _ in range(30):
+        m, n = int(2 ** rng.uniform(4, 11)), int(2 ** rng.uniform(5, 12.5))
+        g = int(rng.choice([16, 32, 64, 128]))
+        k = g * max(1, int(2 ** rng.uniform(6, 12)) // g)
+        packed, s = int4_case(n, k, g, 1, seed=m)
+        w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), to_dev(s), 1, g)
+        x = to_dev(x_case(m, k, "bf16", seed=n), torch.bfloat16)
+        dense = ops.dequant_marlin_cuda("int4", w, sc, n, k, 1, g).double()
+        print(m, n, k, g, flush=True)
+        assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, g), to_np(x.double() @ dense.t()), f"{m}x{n}x{k} g{g}")
