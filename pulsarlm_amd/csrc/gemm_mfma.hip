@@ -204,6 +204,14 @@ int64_t mfma_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool
 }
 
 namespace {
+// Row blocks of an XCD's patch of work tiles. In id order with the row block fastest, an XCD gets the
+// row blocks congruent to its number: with 8 of them one, and every XCD reads all of the weights
+// through its fabric port; with 16 or 32 two or four, which is as good as a patch. Four rows cost the
+// fewest bytes per XCD or nearly for every tile (1, 2, 8 and 16 measured too). id order -> patches of
+// four: W8A8 K 17408, N 5120, M = 333 71 -> 64 us, M = 2048 214 -> 206; int4 K 4096, N 24576,
+// M = 3300 527 -> 505, M = 4096 616 -> 620 (16 row blocks: left in id order).
+int xcd_rows(int m_blocks) { return m_blocks % 16 == 0 ? 0 : std::min(4, m_blocks); }
+
 void launch_mode(plm_format f, bool bf16, const mfma_args& a, int id, bool uniform, bool a8, dim3 grid, hipStream_t s) {
     if (a8) launch_plain_a8(a, bf16, id, grid, s);
     else if (f == PLM_INT4) launch_plain_int4(a, bf16, uniform, id, grid, s);
@@ -241,10 +249,14 @@ int launch_mfma(const char* op, plm_format f, const void* x, bool bf16, const vo
     if (c.tail_halves) {
         // Whole rounds of tall tiles, then the tail's columns of tiles as 128-row halves.
         const int nb_full = (tiles - c.tail_tiles) / c.m_blocks;
+        a.n_blocks = nb_full;
+        a.xcd_rows = xcd_rows(c.m_blocks);
         launch_mode(f, bf16, a, c.shape, uniform, a8, dim3(tiles - c.tail_tiles, 1), s);
         PLM_HIP_LAUNCH_CHECK(op);
         const int mb2 = static_cast<int>(ceil_div(m, kTallHalf.bm()));
         a.m_blocks = mb2;
+        a.n_blocks = c.n_blocks;
+        a.xcd_rows = 0;
         a.tile_base = nb_full * mb2;
         launch_mode(f, bf16, a, kIdH, uniform, a8, dim3((c.n_blocks - nb_full) * mb2, 1), s);
         PLM_HIP_LAUNCH_CHECK(op);
@@ -261,6 +273,7 @@ int launch_mfma(const char* op, plm_format f, const void* x, bool bf16, const vo
         PLM_HIP_LAUNCH_CHECK(op);
         return PLM_OK;
     }
+    a.xcd_rows = xcd_rows(c.m_blocks);
     launch_mode(f, bf16, a, c.shape, uniform, a8, dim3(tiles, c.splits), s);
     PLM_HIP_LAUNCH_CHECK(op);
     return PLM_OK;

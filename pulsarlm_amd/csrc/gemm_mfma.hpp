@@ -57,6 +57,7 @@ struct mfma_args {
     int splits, tiles_per_split;
     int m_blocks, n_blocks;
     int tile_base;  // plain calls: this launch's work tiles start at tile_base
+    int xcd_rows;   // plain calls: row blocks of an XCD's patch of work tiles (0: tiles in id order)
     // A8
     const uint8_t* xq;      // e4m3 [M][ktiles][128], lane-permuted within each tile
     const float* x_scale;   // [M]
@@ -190,8 +191,20 @@ __global__ void __launch_bounds__(WM * WN * 64) mfma_kernel(mfma_args a) {
             c.rows = a.tiles[3 * tile + 2];
             if (c.rows <= 0) return false;  // uniform across the workgroup
         } else {
-            const int mb = item % a.m_blocks;
-            c.nb = item / a.m_blocks;
+            int mb;
+            if (a.xcd_rows > 0) {
+                // Workgroups go round the 8 XCDs by id: each takes one run of the work tiles, which
+                // are ordered in bands of xcd_rows row blocks, row block fastest.
+                const int tiles = a.m_blocks * a.n_blocks, x = item & 7;
+                const int lin = x * (tiles >> 3) + min(x, tiles & 7) + (item >> 3);
+                const int band = lin / (a.xcd_rows * a.n_blocks), first = band * a.xcd_rows;
+                const int rows = min(a.xcd_rows, a.m_blocks - first), in = lin - first * a.n_blocks;
+                c.nb = in / rows;
+                mb = first + in % rows;
+            } else {
+                c.nb = item / a.m_blocks;
+                mb = item % a.m_blocks;
+            }
             c.row0 = mb * BM;
             c.rows = min(BM, a.m - c.row0);
         }

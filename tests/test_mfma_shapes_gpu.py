@@ -83,3 +83,17 @@ def test_random_sizes_by_the_rule(tuning_env):
         dense = ops.dequant_marlin_cuda("int4", w, sc, n, k, 1, g).double()
         print(m, n, k, g, flush=True)
         assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, g), to_np(x.double() @ dense.t()), f"{m}x{n}x{k} g{g}")
+
+
+@pytest.mark.parametrize("m,n,shape", [(5 * 64 - 3, 1016, "R,1"), (9 * 64, 136, "R,2"), (16 * 64, 1016, "R,1"), (17 * 64 + 1, 264, "R,1"),
+                                       (2040, 8440, "X")])
+def test_xcd_patches(m, n, shape, tuning_env):
+    """Every work tile once, for row blocks below, at and past the patch height and at 16 (id order),
+    tile counts that 8 does not divide, and the launch before a tail of half tiles."""
+    packed, s = int4_case(n, K, 128, 1, seed=n)
+    w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), to_dev(s), 1, 128)
+    dense = ops.dequant_marlin_cuda("int4", w, sc, n, K, 1, 128).double()
+    x = to_dev(x_case(m, K, "bf16", seed=m), torch.bfloat16)
+    tuning_env("PLM_MFMA", shape)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128, out=y), to_np(x.double() @ dense.t()), f"{shape} {m}x{n}")
