@@ -109,6 +109,10 @@ __global__ void __launch_bounds__(WM * WN * 64) mfma_kernel(mfma_args a) {
     constexpr int ES = WIDE ? 4 : 2;     // scale element bytes
     // Software-pipelined x fragments (see the K loop), for the one-row tall shapes.
     constexpr bool PIPE_A = UNIFORM && !A8 && WM == 1 && MT >= 8;
+    // The same for W8A8 on the shapes that run one workgroup to a CU (K 4096, N 6144: M = 2048 60.1 ->
+    // 58.3 us, M = 4096 110.3 -> 106.4; K 17408, N 5120, M = 2048 209 -> 205). With two or three
+    // workgroups others fill the waits, and a fixed order costs 2-3 % (K 8192, N 2048, M = 3300).
+    constexpr bool PIPE_A8 = A8 && WM * WN == 8 && NS > 1;
     // Fragments kept a slice ahead: all MT, or 12 for fp8, whose weight tiles already hold
     // two K steps of registers (16 would spill).
     // PERSIST keeps 8 fewer: the item loop needs the registers (the tall tile spills otherwise).
@@ -449,13 +453,42 @@ __global__ void __launch_bounds__(WM * WN * 64) mfma_kernel(mfma_args a) {
                     wv[j][h] = BREG ? wreg[j][h]
                                     : *reinterpret_cast<const u32x4_t*>(sb + (wn * NS + j) * TB + h * 1024 + lane * 16);
 
-            if constexpr (A8) {
+            auto frag_a8 = [&](int i) {
+                const uint8_t* ra = sa + (wm * MT * 16 + i * 16 + col16) * ARB;
+                const u32x4_t a0 = *reinterpret_cast<const u32x4_t*>(ra + (((2 * kq) ^ (col16 & 7)) * 16));
+                const u32x4_t a1 = *reinterpret_cast<const u32x4_t*>(ra + (((2 * kq + 1) ^ (col16 & 7)) * 16));
+                return __builtin_bit_cast(i32x8_t, u32x8_cat(a0, a1));
+            };
+            if constexpr (PIPE_A8) {
+                // AD x fragments are read ahead of their MFMAs, and a product joins its accumulators
+                // (times the block's scale) only after the next row of MFMAs is under way: left to
+                // itself the compiler reads one fragment ahead and waits for it eight times a step.
+                constexpr int AD = MT > 8 ? 2 : 4;
+                i32x8_t af[AD];
+#pragma unroll
+                for (int i = 0; i < AD; ++i) af[i] = frag_a8(i);
+                f32x4_t part[2][NS];
+#pragma unroll
+                for (int i = 0; i <= MT; ++i) {
+#pragma unroll
+                    for (int j = 0; j < NS; ++j) {
+                        if (i < MT)
+                            part[i & 1][j] = mfma16x16x128_fp8(
+                                af[i % AD], __builtin_bit_cast(i32x8_t, u32x8_cat(wv[j][0], wv[j][TB / 1024 - 1])),
+                                f32x4_t{0.f, 0.f, 0.f, 0.f});
+                        if (i > 0)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                acc[i - 1][j][r] = __builtin_fmaf(scale_from_bits<WIDE>(sc[j][0], bf16_scale),
+                                                                  part[(i - 1) & 1][j][r], acc[i - 1][j][r]);
+                        if (j == NS - 1 && i + AD < MT) af[i % AD] = frag_a8(i + AD);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            } else if constexpr (A8) {
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
-                    const uint8_t* ra = sa + (wm * MT * 16 + i * 16 + col16) * ARB;
-                    const u32x4_t a0 = *reinterpret_cast<const u32x4_t*>(ra + (((2 * kq) ^ (col16 & 7)) * 16));
-                    const u32x4_t a1 = *reinterpret_cast<const u32x4_t*>(ra + (((2 * kq + 1) ^ (col16 & 7)) * 16));
-                    const i32x8_t av = __builtin_bit_cast(i32x8_t, u32x8_cat(a0, a1));
+                    const i32x8_t av = frag_a8(i);
 #pragma unroll
                     for (int j = 0; j < NS; ++j) {
                         const i32x8_t bv = __builtin_bit_cast(i32x8_t, u32x8_cat(wv[j][0], wv[j][TB / 1024 - 1]));
