@@ -7,6 +7,7 @@ There is no fallback: every op in this package runs the HIP library.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -67,12 +68,31 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+# Sizes that depend on the call's shape alone; a ctypes call costs about as long as a small
+# kernel's launch, so the last shapes' are kept.
+@functools.lru_cache(maxsize=1024)
+def weight_bytes(fmt: int, n: int, k: int) -> int:
+    return load().plm_weight_bytes(fmt, n, k)
+
+
+@functools.lru_cache(maxsize=1024)
+def gemm_workspace_bytes(fmt: int, m: int, n: int, k: int) -> int:
+    return load().plm_gemm_workspace_bytes(fmt, m, n, k)
+
+
+@functools.lru_cache(maxsize=1024)
+def gemm_w8a8_workspace_bytes(m: int, n: int, k: int) -> int:
+    return load().plm_gemm_w8a8_workspace_bytes(m, n, k)
+
+
 def reload_tuning() -> None:
     """Make the library re-read its PLM_* measurement knobs from the environment (it parses
     them once per process otherwise). An internal hook for tests, not part of the C ABI."""
     fn = load().plm_internal_reload_tuning
     fn.restype, fn.argtypes = None, []
     fn()
+    gemm_workspace_bytes.cache_clear()  # the plans follow the knobs
+    gemm_w8a8_workspace_bytes.cache_clear()
 
 
 def check(rc: int) -> None:
