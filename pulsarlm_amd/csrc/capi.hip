@@ -1,7 +1,8 @@
 // C-ABI GEMM entry points: argument checks (mirroring gemm<fmt>,
 // pulsarlm-core/src/kernels/marlin.cu:538-576) and dispatch between the decode
 // kernels (M <= 16, the reference's small_m switch at marlin.cu:577, and up to 32 rows
-// where measured faster) and the MFMA kernel.
+// where measured faster), the rows kernel (up to 128 rows where measured faster than
+// either) and the MFMA kernel.
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>

@@ -9,12 +9,9 @@
 //
 // gfx950 design:
 // * Workgroup tile (WM*MT*16) x (WN*NS*16) over 128-wide K steps; WM x WN wavefronts,
-//   each owning MT x NS tiles of v_mfma_f32_16x16x32 (bf16/fp16) -- 128 x 64 per
-//   wavefront in the large configuration (256 x 128 per workgroup, one wavefront per
-//   SIMD with the full 512 registers), so each dequantized weight feeds 8 MFMAs and the
-//   dequant VALU work is about half the MFMA time, interleaved with it. The int4 256 x 256
-//   tile for plain calls uses 8 wavefronts of 256 x 32 each, so every strip is dequantized
-//   by one wavefront only (a 2 x 4 wavefront grid would dequantize each strip twice).
+//   each owning MT x NS tiles of v_mfma_f32_16x16x32 (bf16/fp16). Most shapes have one row
+//   of wavefronts, so every strip is dequantized by one wavefront only and each dequantized
+//   weight feeds MT MFMAs (a second row of wavefronts would dequantize each strip twice).
 // * The x tile and the packed weight tiles (1 KiB int4 / 2 KiB fp8 per 16-column strip,
 //   copied verbatim from the plm layout) go from HBM straight into LDS with buffer loads to
 //   LDS (no register staging), double-buffered: the next K step's loads land in one stage
