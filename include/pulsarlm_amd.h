@@ -116,7 +116,7 @@ int64_t plm_gemm_workspace_bytes(plm_format format, int64_t m, int64_t n, int64_
  * (ops.hpp:316-332, marlin.cu:538-597,631-651).
  * The smallest M runs the bandwidth-first decode kernels, up to 128 rows the rows kernel where
  * measured faster, larger M the MFMA kernel.
- * M == 0 or N == 0 returns PLM_OK without touching y.
+ * M == 0 or N == 0 returns PLM_OK without touching y; K == 0 sets y to zero.
  */
 int plm_gemm(plm_format format, const void* x, plm_dtype x_dtype,
              const void* weight, const void* scale, plm_dtype scale_dtype,

@@ -69,12 +69,25 @@ int check_gemm(const char* op, plm_format f, const void* x, plm_dtype x_dtype, c
     return PLM_OK;
 }
 
+// y = 0 for K == 0 (a sum over nothing): no K tile exists to plan a kernel for. Element stores,
+// since y need only be 2-byte aligned.
+__global__ void __launch_bounds__(256) zero_output_kernel(uint16_t* __restrict__ y, int64_t n) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256) y[i] = 0;
+}
+int zero_output(const char* op, void* y, int64_t m, int64_t n, hipStream_t s) {
+    const int64_t blocks = std::min<int64_t>(ceil_div(m * n, 256), 16 * static_cast<int64_t>(cu_count()));
+    zero_output_kernel<<<static_cast<unsigned>(blocks), 256, 0, s>>>(static_cast<uint16_t*>(y), m * n);
+    PLM_HIP_LAUNCH_CHECK(op);
+    return PLM_OK;
+}
+
 // Checked arguments to a kernel: the rows kernel where its rule takes the call, else the decode
 // or MFMA kernels. A call is refused for its workspace by those two paths' needs alone: one
 // that is too small for the rows kernel's K split only keeps the call from it.
 int run_gemm(const char* op, plm_format f, const void* x, bool bf16, const void* w, const void* scale, plm_dtype scale_dtype,
              int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size, void* y, void* workspace,
              size_t workspace_bytes, hipStream_t s) {
+    if (k == 0) return zero_output(op, y, m, n, s);
     const bool decode = use_decode(m, n);
     const int64_t need = decode ? decode_workspace_bytes(f, m, n, k) : mfma_contract(f, m, n, k, false);
     const bool enough = need == 0 || (workspace != nullptr && static_cast<int64_t>(workspace_bytes) >= need);
@@ -167,6 +180,7 @@ int plm_gemm_w8a8(const void* x, plm_dtype x_dtype, const void* weight, const vo
         return rc;
     PLM_CHECK_ARG(group_size % kTileK == 0, op, "group_size must be a multiple of 128 for the fp8 MFMA");
     if (m == 0 || n == 0) return PLM_OK;
+    if (k == 0) return zero_output(op, y, m, n, as_stream(stream));
     const w8a8_ws l = w8a8_layout(m, n, k, workspace != nullptr ? static_cast<int64_t>(workspace_bytes) : 0);
     if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < l.total) {
         set_error(op, "workspace of %lld bytes required, %zu given", static_cast<long long>(l.total), workspace_bytes);

@@ -3,7 +3,11 @@ every declared symbol, sizes agree with the layout, and argument errors are
 reported with the op's name before any device work (no GPU needed)."""
 
 import ctypes
+import os
 import re
+import subprocess
+import sys
+import textwrap
 from pathlib import Path
 
 import pytest
@@ -74,6 +78,27 @@ def test_empty_gemm_is_ok_without_device_work():
     rc = lib.plm_gemm(_lib.PLM_INT4, None, _lib.PLM_BF16, None, None, _lib.PLM_FP16, 0, 64, 128, 1, 128, None, None, 0,
                       None)
     assert rc == _lib.PLM_OK
+
+
+def test_zero_k_reaches_the_launch():
+    """K == 0 plans no kernel (there is no K tile to divide by): the call gets as far as its launch, which
+    has no device here. In a process of its own, as a host fault would end it."""
+    script = textwrap.dedent("""
+        import ctypes
+        from pulsarlm_amd import _lib
+        lib, d = _lib.load(), ctypes.c_void_p(256)
+        for m in (1, 16, 24, 48, 300):
+            for n in (64, 8192):
+                for fmt in (_lib.PLM_INT4, _lib.PLM_FP8):
+                    rc = lib.plm_gemm(fmt, d, _lib.PLM_BF16, d, d, _lib.PLM_FP32, m, n, 0, 1, 128, d, None, 0, None)
+                    assert rc == _lib.PLM_ERR_HIP, rc
+                rc = lib.plm_gemm_w8a8(d, _lib.PLM_BF16, d, d, _lib.PLM_FP32, m, n, 0, 1, 128, d, None, 0, None)
+                assert rc == _lib.PLM_ERR_HIP, rc
+        print("REACHED")
+    """)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")
+    res = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, cwd=HEADER.parents[1], env=env)
+    assert res.returncode == 0 and "REACHED" in res.stdout, res.stdout + res.stderr
 
 
 def test_repack_argument_errors():

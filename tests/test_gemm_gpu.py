@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from pulsarlm_amd import ops
+from pulsarlm_amd import _lib, ops
 from tests._util import TDT, assert_close, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
@@ -144,6 +144,22 @@ def test_int4_gemm_below_one_k_tile(m, n, k):
     x = x_case(m, k, "bf16", seed=m + k)
     y = ops.gemm_int4_marlin_cuda(to_dev(x, torch.bfloat16), w, sc, n, 1, g)
     assert_close(y, O.gemm_ref(x, O.dequant_int4(packed, s, 1, g), None), f"m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m,n", [(1, 64), (16, 8200), (24, 40), (48, 1000), (300, 1001)])
+def test_zero_k_gives_zeros(m, n):
+    """K == 0: every output is the sum over nothing, from plm_gemm, plm_gemm_noalloc and plm_gemm_w8a8, and
+    nothing past y is written."""
+    lib = _lib.load()
+    some = torch.empty(256, dtype=torch.uint8, device="cuda").data_ptr()
+    st = torch.cuda.current_stream().cuda_stream
+    for fn, args in (("plm_gemm", (_lib.PLM_INT4,)), ("plm_gemm", (_lib.PLM_FP8,)), ("plm_gemm_noalloc", (_lib.PLM_INT4,)),
+                     ("plm_gemm_w8a8", ())):
+        buf = torch.ones(m * n + 8, dtype=torch.bfloat16, device="cuda")
+        tail = () if fn == "plm_gemm_noalloc" else (None, 0)
+        rc = getattr(lib, fn)(*args, some, _lib.PLM_BF16, some, some, _lib.PLM_FP32, m, n, 0, 1, 128, buf[1:].data_ptr(), *tail, st)
+        assert rc == _lib.PLM_OK, (fn, lib.plm_last_error())
+        assert int((buf == 0).sum()) == m * n and buf[0] == 1 and bool((buf[m * n + 1:] == 1).all()), fn
 
 
 @pytest.mark.parametrize("m", [1, 3, 4, 8, 13, 16])
