@@ -172,22 +172,45 @@ bool use_rows(plm_format f, int64_t m, int64_t n, int64_t k, int64_t group_size,
     return m > 4 || strips != cus || k > 12288;
 }
 
+// A call as the rows kernel would run it; `taken` is false where it does not take the call (the
+// workspace aside, which launch_rows looks at).
+struct rows_call {
+    bool taken = false;
+    rows_plan p;
+    layout_dims d;
+    int scm;
+    int64_t s_stage, lds;
+};
+
+rows_call resolve_rows(plm_format f, plm_dtype scale_dtype, int64_t m, int64_t n, int64_t k, int64_t block_n, int64_t group_size) {
+    rows_call c;
+    const bool sub = group_size % kTileK != 0;
+    if (m > kRowsMaxM || k > kRowsMaxK || (f == PLM_FP8 && sub) ||
+        !use_rows(f, m, n, k, group_size, decode_rr_takes(f, m, n, k, block_n, group_size, scale_dtype)))
+        return c;
+    c.p = plan_rows(f, m, n, k);
+    if (c.p.rb == 0) return c;
+    c.d = make_dims(n, k, block_n, group_size);
+    c.scm = c.d.scale_cols == 16 ? (scale_dtype == PLM_FP32 ? 1 : 0) : (scale_dtype == PLM_FP32 ? 2 : -1);
+    if (f == PLM_INT4 ? c.scm != 0 && c.scm != 1 : c.scm != 1 && c.scm != 2) return c;  // no instantiation
+    const int64_t eb = c.d.scale_cols * dtype_size(scale_dtype);
+    if (c.d.strips * c.d.groups * eb >= kOOB) return c;
+    const int64_t span = c.p.splits == 1 ? c.d.groups
+                                         : std::min<int64_t>(c.d.groups, ceil_div(int64_t{c.p.tiles_per_split} * kTileK, group_size) + 1);
+    c.s_stage = round_up(span * eb, 256);
+    c.lds = rows_lds_bytes(c.p.rb, c.p.sg, c.s_stage);
+    c.taken = c.lds <= 160 * 1024;
+    return c;
+}
+
 // Returns false, with nothing launched, where the rows kernel does not take the call.
 bool launch_rows(plm_format f, const void* x, bool bf16, const void* w, const void* scale, plm_dtype scale_dtype, int64_t m,
                  int64_t n, int64_t k, int64_t block_n, int64_t group_size, void* y, void* workspace, size_t workspace_bytes,
                  hipStream_t s) {
-    if (m > kRowsMaxM || k > kRowsMaxK || !use_rows(f, m, n, k, group_size, decode_rr_takes(f, m, n, k, block_n, group_size, scale_dtype)))
-        return false;
-    const rows_plan p = plan_rows(f, m, n, k);
-    if (p.rb == 0) return false;
-    const layout_dims d = make_dims(n, k, block_n, group_size);
-    const int scm = d.scale_cols == 16 ? (scale_dtype == PLM_FP32 ? 1 : 0) : (scale_dtype == PLM_FP32 ? 2 : -1);
-    const int64_t eb = d.scale_cols * dtype_size(scale_dtype);
-    if (scm < 0 || d.strips * d.groups * eb >= kOOB) return false;
-    const int64_t span = p.splits == 1 ? d.groups : std::min<int64_t>(d.groups, ceil_div(int64_t{p.tiles_per_split} * kTileK, group_size) + 1);
-    const int64_t s_stage = round_up(span * eb, 256);
-    const int64_t lds = rows_lds_bytes(p.rb, p.sg, s_stage);
-    if (lds > 160 * 1024) return false;
+    const rows_call c = resolve_rows(f, scale_dtype, m, n, k, block_n, group_size);
+    if (!c.taken) return false;
+    const rows_plan& p = c.p;
+    const layout_dims& d = c.d;
     const int64_t need = rows_need(p);
     if (need > 0 && (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need)) return false;
     rows_args a{};
@@ -204,11 +227,26 @@ bool launch_rows(plm_format f, const void* x, bool bf16, const void* w, const vo
     a.scale_dtype = scale_dtype;
     const uint64_t g16 = static_cast<uint64_t>(group_size) / 16;
     a.group_magic = static_cast<uint32_t>(((uint64_t{1} << 31) + g16 - 1) / g16);
-    a.s_stage = static_cast<int>(s_stage);
+    a.s_stage = static_cast<int>(c.s_stage);
     const dim3 grid(static_cast<unsigned>(p.m_blocks * p.n_blocks), static_cast<unsigned>(p.splits));
     const bool sub = group_size % kTileK != 0;
-    return f == PLM_INT4 ? launch_rows_shape<PLM_INT4>(a, bf16, scm, sub, p.rb, p.sg, grid, static_cast<size_t>(lds), s)
-                         : launch_rows_shape<PLM_FP8>(a, bf16, scm, sub, p.rb, p.sg, grid, static_cast<size_t>(lds), s);
+    return f == PLM_INT4 ? launch_rows_shape<PLM_INT4>(a, bf16, c.scm, sub, p.rb, p.sg, grid, static_cast<size_t>(c.lds), s)
+                         : launch_rows_shape<PLM_FP8>(a, bf16, c.scm, sub, p.rb, p.sg, grid, static_cast<size_t>(c.lds), s);
 }
 
 }  // namespace plm
+
+extern "C" {
+// Not part of the public ABI (include/pulsarlm_amd.h): how plm_gemm would run a call on the rows kernel
+// given enough workspace, for the tests that aim at it. out[0..5]: taken (0/1), row blocks and strips
+// of a workgroup, workgroups over rows and columns, K splits.
+__attribute__((visibility("default"))) void plm_internal_rows_plan(int format, int64_t m, int64_t n, int64_t k, int64_t block_n,
+                                                                  int64_t group_size, int scale_dtype, int32_t* out) {
+    using namespace plm;
+    const rows_call c = resolve_rows(static_cast<plm_format>(format), static_cast<plm_dtype>(scale_dtype), m, n, k, block_n, group_size);
+    out[0] = c.taken ? 1 : 0;
+    out[1] = c.p.rb, out[2] = c.p.sg;
+    out[3] = c.p.m_blocks, out[4] = c.p.n_blocks;
+    out[5] = c.p.splits;
+}
+}  // extern "C"
