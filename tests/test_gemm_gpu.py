@@ -13,7 +13,7 @@ import torch
 
 from oracle import oracle as O
 from pulsarlm_amd import _lib, ops
-from tests._util import TDT, assert_close, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
+from tests._util import TDT, assert_close, force_mfma, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
 
@@ -368,7 +368,7 @@ def test_mfma_epilogue_store_forms(n, y_shift, tuning_env):
     aligned call's result on the same shape bit for bit, and every row must match the fp32
     reference."""
     m, k = 512, 512  # 8 tall tiles, K not split (the split-K kernels keep the 2-byte stores)
-    tuning_env("PLM_MFMA", "X")
+    force_mfma(tuning_env, "int4", m, n, k, "X", 1)
     x, packed, s = _full_case(m, k, n, seed=n + y_shift)
     w, sc = ops.repack_int4_marlin_cuda(packed, s, 1, 128)
     wd = ops.dequant_marlin_cuda("int4", w, sc, n, k, 1, 128)

@@ -9,13 +9,19 @@ import torch
 
 from oracle import oracle as O
 from pulsarlm_amd import ops
-from tests._util import TDT, assert_close, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
+from tests._util import TDT, assert_close, force_mfma, fp8_case, int4_case, mfma_plan, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
 
-# N = 1016: the last strip is half empty and no shape's strips divide its 64; K = 1152: 9 K tiles.
-N, K = 1016, 1152
+# N = 1016: the last strip is half empty and no shape's strips divide its 64; K = 3072: 24 K tiles, so that
+# splits of 5 (the last one a tile shorter) and 8 exist.
+N, K = 1016, 3072
 ROWS = {"R": 64, "W": 256, "X": 256, "Q": 64, "H": 128, "B": 128, "C": 96, "D": 112, "F": 96, "A": 128, "G": 256, "S": 128}
+
+
+def _splits(shape, m):
+    """8 where the plan allows it: its limits are the partial sums' bytes and the tiles per CU."""
+    return (1, 5, 8 if m <= ROWS[shape] + 1 else 4)
 
 
 @pytest.fixture(autouse=True)
@@ -33,8 +39,8 @@ def test_int4_shapes(shape, g, dtype, sdt, tuning_env):
     for m in (33, ROWS[shape] - 1, ROWS[shape] + 1, 3 * ROWS[shape] + 17):
         x = to_dev(x_case(m, K, dtype, seed=m), TDT[dtype])
         ref = to_np(x.double() @ dense.t())
-        for splits in (1, 3, 8):
-            tuning_env("PLM_MFMA", f"{shape},{splits}")
+        for splits in _splits(shape, m):
+            force_mfma(tuning_env, "int4", m, N, K, shape, splits)
             y = ops.gemm_int4_marlin_cuda(x, w, sc, N, 1, g)
             assert_close(y, ref, f"{shape} m={m} splits={splits}")
             assert torch.equal(y, ops.gemm_int4_marlin_cuda(x, w, sc, N, 1, g)), "not deterministic"
@@ -49,8 +55,8 @@ def test_fp8_shapes(shape, block_n, dtype, tuning_env):
     for m in (33, ROWS[shape] - 1, ROWS[shape] + 1, 2 * ROWS[shape] + 17):
         x = to_dev(O.round_to(x_case(m, K, dtype, seed=m) * np.float32(0.05), dtype), TDT[dtype])
         ref = to_np(x.double() @ dense.t())
-        for splits in (1, 3, 8):
-            tuning_env("PLM_MFMA", f"{shape},{splits}")
+        for splits in _splits(shape, m):
+            force_mfma(tuning_env, "fp8", m, N, K, shape, splits)
             assert_close(ops.gemm_fp8_marlin_cuda(x, w, sc, N, block_n, 128), ref, f"{shape} m={m} splits={splits}")
 
 
@@ -63,8 +69,8 @@ def test_w8a8_shapes(shape, tuning_env):
         x = x_case(m, K, "bf16", seed=m)
         xc, xs = O.quantize_per_token_e4m3(x)
         ref = O.gemm_w8a8_ref(xc, xs, codes, scale, 128, 128, dtype=None)
-        for splits in (1, 3, 8):
-            tuning_env("PLM_MFMA", f"{shape},{splits}")
+        for splits in _splits(shape, m):
+            force_mfma(tuning_env, "w8a8", m, N, K, shape, splits)
             y = ops.gemm_fp8_w8a8_cuda(to_dev(x, torch.bfloat16), w, sc, N, 128, 128)
             assert_close(y, ref, f"{shape} m={m} splits={splits}")
 
@@ -85,15 +91,21 @@ def test_random_sizes_by_the_rule(tuning_env):
         assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, g), to_np(x.double() @ dense.t()), f"{m}x{n}x{k} g{g}")
 
 
-@pytest.mark.parametrize("m,n,shape", [(5 * 64 - 3, 1016, "R,1"), (9 * 64, 136, "R,2"), (16 * 64, 1016, "R,1"), (17 * 64 + 1, 264, "R,1"),
-                                       (2040, 8440, "X")])
-def test_xcd_patches(m, n, shape, tuning_env):
+@pytest.mark.parametrize("m,n,shape,splits", [(5 * 64 - 3, 1016, "R", 1), (9 * 64, 136, "R", 2), (16 * 64, 1016, "R", 1),
+                                              (17 * 64 + 1, 264, "R", 1), (2040, 8440, "X", 0)])
+def test_xcd_patches(m, n, shape, splits, tuning_env):
     """Every work tile once, for row blocks below, at and past the patch height and at 16 (id order),
     tile counts that 8 does not divide, and the launch before a tail of half tiles."""
-    packed, s = int4_case(n, K, 128, 1, seed=n)
+    k = 1152
+    packed, s = int4_case(n, k, 128, 1, seed=n)
     w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), to_dev(s), 1, 128)
-    dense = ops.dequant_marlin_cuda("int4", w, sc, n, K, 1, 128).double()
-    x = to_dev(x_case(m, K, "bf16", seed=m), torch.bfloat16)
-    tuning_env("PLM_MFMA", shape)
+    dense = ops.dequant_marlin_cuda("int4", w, sc, n, k, 1, 128).double()
+    x = to_dev(x_case(m, k, "bf16", seed=m), torch.bfloat16)
+    if splits:
+        force_mfma(tuning_env, "int4", m, n, k, shape, splits)
+    else:
+        tuning_env("PLM_MFMA", shape)
+        p = mfma_plan("int4", m, n, k)
+        assert p["tile"] == (256, 256) and p["halves"], p
     y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
     assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128, out=y), to_np(x.double() @ dense.t()), f"{shape} {m}x{n}")

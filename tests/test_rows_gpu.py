@@ -10,7 +10,7 @@ import torch
 
 from oracle import oracle as O
 from pulsarlm_amd import ops
-from tests._util import TDT, assert_close, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
+from tests._util import TDT, assert_close, force_rows, fp8_case, int4_case, rows_plan, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
 
@@ -29,13 +29,13 @@ def _int4(n, k, g, sdt, seed):
 # Row blocks of one to four (and two row blocks of them), one to four strips and K splits, on a
 # strip count that no group divides (N = 1016: 63.5 strips, the last one half empty).
 @pytest.mark.parametrize("m", [5, 16, 17, 33, 48, 49, 64, 65, 97, 128])
-@pytest.mark.parametrize("shape", ["1,1", "2,3", "3,2", "4,8", "4,1"])
+@pytest.mark.parametrize("shape", [(1, 1), (2, 3), (3, 2), (4, 8), (4, 1), (1, 4)])
 def test_int4_shapes_and_splits(m, shape, tuning_env):
-    n, k = 1016, 2176  # 17 K tiles: the wavefronts hold one to three, in splits down to none
+    n, k = 1016, 2944  # 23 K tiles: the wavefronts hold two or three, in splits down to none
     packed, s, (w, sc) = _int4(n, k, 128, "fp16", seed=m)
     x = x_case(m, k, "bf16", seed=m)
     ref = O.gemm_ref(x, O.dequant_int4(packed, s, 1, 128), None)
-    tuning_env("PLM_ROWS", shape)
+    force_rows(tuning_env, "int4", m, n, k, 1, 128, "fp16", *shape)
     xd = to_dev(x, torch.bfloat16)
     a = ops.gemm_int4_marlin_cuda(xd, w, sc, n, 1, 128)
     assert_close(a, ref, f"m={m} rows {shape}")
@@ -50,8 +50,10 @@ def test_int4_shapes_and_splits(m, shape, tuning_env):
 @pytest.mark.parametrize("g,k", [(16, 144), (32, 4128), (48, 1008), (64, 2112), (80, 1040), (112, 896), (128, 128),
                                  (256, 2560), (384, 2688)])
 @pytest.mark.parametrize("sdt,dtype", [("fp16", "fp16"), ("fp32", "bf16"), ("bf16", "bf16")])
-def test_int4_groups_and_k_tails(m, g, k, sdt, dtype):
+def test_int4_groups_and_k_tails(m, g, k, sdt, dtype, tuning_env):
     n = 520
+    tuning_env("PLM_ROWS", "1")
+    assert rows_plan("int4", m, n, k, 1, g, sdt) is not None
     packed, s, (w, sc) = _int4(n, k, g, sdt, seed=g + m)
     x = x_case(m, k, dtype, seed=k)
     y = ops.gemm_int4_marlin_cuda(to_dev(x, TDT[dtype]), w, sc, n, 1, g)
@@ -60,23 +62,27 @@ def test_int4_groups_and_k_tails(m, g, k, sdt, dtype):
 
 @pytest.mark.parametrize("m", [4, 16, 31, 48, 64, 80])
 @pytest.mark.parametrize("block_n,dtype", [(128, "bf16"), (1, "fp16")])
-@pytest.mark.parametrize("shape", ["1,1", "2,2", "3,1", "4,4"])
-def test_fp8_shapes(m, block_n, dtype, shape, tuning_env):
-    n, k = 7176, 2304  # above 1.5 strips per CU, so that every row count takes the rows kernel
+@pytest.mark.parametrize("n,k,shape", [(7176, 2304, (1, 1)), (7176, 2304, (2, 2)), (7176, 2304, (3, 1)), (7176, 2304, (4, 3)),
+                                       (1016, 2944, (4, 8))])
+def test_fp8_shapes(m, block_n, dtype, n, k, shape, tuning_env):
     codes, s = fp8_case(n, k, 128, block_n, seed=m)
     w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), scale_tensor(s), block_n, 128)
     x = x_case(m, k, dtype, seed=m) * np.float32(0.05)
     x = O.round_to(x, dtype)
-    tuning_env("PLM_ROWS", shape)
+    force_rows(tuning_env, "fp8", m, n, k, block_n, 128, "fp32", *shape)
     xd = to_dev(x, TDT[dtype])
     y = ops.gemm_fp8_marlin_cuda(xd, w, sc, n, block_n, 128)
     dense = ops.dequant_marlin_cuda("fp8", w, sc, n, k, block_n, 128, TDT[dtype])  # pinned to the oracle elsewhere
-    assert_close(y, to_np(xd.double() @ dense.double().t()), f"m={m} bn={block_n} {shape}")
+    ref = to_np(xd.double() @ dense.double().t())
+    assert_close(y, ref, f"m={m} bn={block_n} {shape}")
+    tuning_env("PLM_ROWS", "0")
+    assert_close(ops.gemm_fp8_marlin_cuda(xd, w, sc, n, block_n, 128), ref, f"m={m} bn={block_n} without the rows kernel")
 
 
 def test_rows_beside_nan_and_inf():
     """A non-finite value in one row stays in that row, and x past the last row is never read."""
     m, n, k = 20, 512, 4096
+    assert rows_plan("int4", m, n, k, 1, 128, "fp16") is not None
     packed, s, (w, sc) = _int4(n, k, 128, "fp16", seed=3)
     x = x_case(64, k, "bf16", seed=4)
     big = to_dev(x, torch.bfloat16)
@@ -92,9 +98,11 @@ def test_rows_beside_nan_and_inf():
     assert torch.equal(y[keep], clean[keep])
 
 
-@pytest.mark.parametrize("fmt,m,n,k", [("int4", 48, 4096, 4096), ("int4", 100, 4096, 12288), ("fp8", 16, 5120, 17408)])
+@pytest.mark.parametrize("fmt,m,n,k", [("int4", 48, 1024, 4096), ("int4", 100, 2048, 8192), ("fp8", 16, 5120, 17408)])
 def test_split_rows_graph_replays_match_eager(fmt, m, n, k):
     """Calls whose plan splits K, captured: the arrival counters are left zero by every call."""
+    p = rows_plan(fmt, m, n, k, 1 if fmt == "int4" else 128, 128, "fp16" if fmt == "int4" else "fp32")
+    assert p is not None and p["splits"] > 1, p
     rng = np.random.default_rng(5)
     x = to_dev(rng.standard_normal((m, k)).astype(np.float32), torch.bfloat16)
     if fmt == "int4":
