@@ -43,3 +43,9 @@ def tuning_env(monkeypatch):
     yield set_knob
     monkeypatch.undo()
     _lib.reload_tuning()
+
+
+@pytest.fixture(params=[None, "0"], ids=["rule", "no_rows"])
+def with_and_without_rows(request, tuning_env):
+    """Calls up to 128 rows by the dispatch rule, and without the rows kernel, on the decode and MFMA kernels."""
+    tuning_env("PLM_ROWS", request.param)

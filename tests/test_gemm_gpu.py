@@ -73,9 +73,9 @@ def test_dequant_bit_exact(fmt, dtype, block_n):
 @pytest.mark.parametrize("block_n", [1, 128])
 @pytest.mark.parametrize("fmt", ["int4", "fp8"])
 @pytest.mark.parametrize("g", [16, 48, 32, 128])
-def test_identity_gemm_exact(fmt, dtype, block_n, g):
+def test_identity_gemm_exact(fmt, dtype, block_n, g, with_and_without_rows):
     """test_marlin.cpp:54-78: y = I_k @ dequant(W)^T must equal dequant(W)^T exactly,
-    through the MFMA path (M = K) and the decode path (16-row and 1-row slices)."""
+    through the MFMA path (M = K) and the decode and rows kernels (16-row and 1-row slices)."""
     n, k = N, 144 if g in (16, 48) else 256
     if fmt == "int4":
         packed, s = int4_case(n, k, g, block_n, seed=4, scale_dtype=np.float32, scale_kind="test")
@@ -123,7 +123,7 @@ def test_fp8_gemm_reference_shape(m, dtype):
 
 @pytest.mark.parametrize("m", [1, 4, 16, 64, 256])
 @pytest.mark.parametrize("g", [32, 64, 128, 256])
-def test_int4_gemm_group_sizes(m, g):
+def test_int4_gemm_group_sizes(m, g, with_and_without_rows):
     n, k = 520, 1024
     packed, s = int4_case(n, k, g, 1, seed=g)
     w, sc = _repack_int4(packed, s, 1, g)
@@ -134,10 +134,10 @@ def test_int4_gemm_group_sizes(m, g):
 
 @pytest.mark.parametrize("m", [1, 17, 40, 300])
 @pytest.mark.parametrize("n,k", [(8, 16), (40, 32), (24, 48), (200, 16)])
-def test_int4_gemm_below_one_k_tile(m, n, k):
+def test_int4_gemm_below_one_k_tile(m, n, k, with_and_without_rows):
     """K below one 128-wide tile (16-wide groups, the reference test's group size) and N below
-    or not a multiple of a 16-column strip, on the decode kernels (M <= 32) and the MFMA
-    kernel (M > 32): the partial K tile and the partial strip read as zero."""
+    or not a multiple of a 16-column strip, on the rows kernel, the decode kernels (M <= 32) and the
+    MFMA kernel: the partial K tile and the partial strip read as zero."""
     g = 16
     packed, s = int4_case(n, k, g, 1, seed=n + k)
     w, sc = _repack_int4(packed, s, 1, g)
@@ -164,8 +164,8 @@ def test_zero_k_gives_zeros(m, n):
 
 @pytest.mark.parametrize("m", [1, 3, 4, 8, 13, 16])
 @pytest.mark.parametrize("case", ["fp16s-bf16x", "fp32s-bf16x", "bf16s-fp16x", "fp32s-strip", "g256"])
-def test_decode_kernel_variants(m, case):
-    """The M <= 16 decode kernels across scale layouts, activation dtypes and a ragged strip
+def test_decode_kernel_variants(m, case, with_and_without_rows):
+    """The M <= 16 kernels across scale layouts, activation dtypes and a ragged strip
     count (N = 8200: 513 strips, so strip groups of 2, 3 or more end in a partial group)."""
     n, k, g, block_n, dtype = 8200, 512, 128, 1, "bf16"
     sdt = np.float16
@@ -223,19 +223,21 @@ def test_deterministic_across_calls():
 
 
 @pytest.mark.parametrize("case", [
-    ("int4", 16, 12288, 4096),  # decode kernel with a K split across workgroups
+    ("int4", 16, 12288, 4096),  # rows kernel
+    ("int4", 16, 12288, 4096, "no rows kernel"),  # decode kernel with a K split across workgroups
     ("int4", 256, 4096, 4096),  # MFMA kernel with a K split (fewer tiles than CUs)
     ("int4", 4096, 4096, 6144),  # MFMA kernel: whole rounds, then the tail as 128-row halves
     ("fp8", 2048, 5120, 34816),  # fp8 W8A16 tall tiles: whole rounds, then the K-split tail launch
-    ("fp8", 16, 5120, 7168),  # fp8 W8A16 decode: two strips on 8 wavefronts, K split in two
+    ("fp8", 16, 5120, 7168, "no rows kernel"),  # fp8 W8A16 decode: two strips on 8 wavefronts, K split in two
     ("w8a8", 16, 5120, 5120),  # per-token quantizer, then the W8A8 decode kernel
     ("w8a8", 2, 5120, 5120),  # the W8A8 decode kernel with the quantizer fused in
 ])
-def test_gemm_graph_replays_match_eager(case):
+def test_gemm_graph_replays_match_eager(case, tuning_env):
     """plm_gemm captured into a graph: the split-K arrival counters are reset by the last
     workgroup of every call, so each replay (with eager calls between them) must equal the
     eager result bit for bit."""
-    fmt, m, k, n = case
+    fmt, m, k, n = case[:4]
+    tuning_env("PLM_ROWS", "0" if len(case) > 4 else None)
     print(f"graph replay case {case}", flush=True)
     rng = np.random.default_rng(61)
     xd = torch.from_numpy(rng.standard_normal((m, k), dtype=np.float32)).to("cuda").to(torch.bfloat16)
@@ -382,9 +384,9 @@ def test_mfma_epilogue_store_forms(n, y_shift, tuning_env):
     assert torch.equal(y, ref)
 
 
-def test_decode_and_mfma_kernels_agree():
-    """M=16 and M=32 run the decode kernels (one and two 16-row blocks), M=33 the MFMA
-    kernel; their common rows must agree to the GEMM tolerance (each is checked against the
+def test_decode_and_mfma_kernels_agree(with_and_without_rows):
+    """Without the rows kernel M=16 and M=32 run the decode kernels (one and two 16-row blocks) and
+    M=33 the MFMA kernel; their common rows must agree to the GEMM tolerance (each is checked against the
     oracle elsewhere)."""
     k, n = 12288, 4096
     x, packed, s = _full_case(33, k, n, seed=5)
@@ -398,10 +400,10 @@ def test_decode_and_mfma_kernels_agree():
 
 @pytest.mark.parametrize("m", [17, 20, 24, 28, 31, 32])
 @pytest.mark.parametrize("shape", [(4096, 6144), (4096, 4096), (4096, 24576), (12288, 4096)])
-def test_two_row_block_decode(shape, m):
-    """17 to 32 rows: the decode kernels with two 16-row MFMA blocks per dequantized weight
-    fragment (gate_up above 24 rows goes to the MFMA kernel), rows past M of the second
-    block never stored."""
+def test_two_row_block_decode(shape, m, with_and_without_rows):
+    """17 to 32 rows, by the rule and, without the rows kernel, on the decode kernels with two 16-row
+    MFMA blocks per dequantized weight fragment (gate_up above 24 rows goes to the MFMA kernel):
+    rows past M of the second block are never stored."""
     k, n = shape
     x, packed, s = O.make_w4a16(m, n, k, 128, seed=k + n + m)
     w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), to_dev(s), 1, 128)
@@ -411,7 +413,7 @@ def test_two_row_block_decode(shape, m):
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("case", ["fp16s", "fp32s-strip", "g256", "g64", "k-tail"])
-def test_two_row_block_decode_variants(case, dtype):
+def test_two_row_block_decode_variants(case, dtype, with_and_without_rows):
     """Two row blocks across scale layouts, groups below and above one K tile, fp16 x, a
     ragged strip count (N = 8200) and a partial last K tile (K = 400, 16-wide groups)."""
     m, n, k, g, block_n, sdt = 23, 8200, 512, 128, 1, np.float16
@@ -433,7 +435,7 @@ def test_two_row_block_decode_variants(case, dtype):
 
 @pytest.mark.parametrize("m", [1, 4, 7, 16, 17, 32])
 @pytest.mark.parametrize("n,k,g", [(16, 128, 128), (48, 128, 128), (40, 256, 256), (1000, 384, 128)])
-def test_decode_small_k_and_narrow_n(m, n, k, g):
+def test_decode_small_k_and_narrow_n(m, n, k, g, with_and_without_rows):
     """Decode kernels where most wavefronts of a workgroup own no K tile (K of 1-3 tiles),
     a single strip (N = 16) and a 256-wide scale group spanning two tiles."""
     packed, s = int4_case(n, k, g, 1, seed=n + k + m)
@@ -446,9 +448,10 @@ def test_decode_small_k_and_narrow_n(m, n, k, g):
 @pytest.mark.parametrize("m", [1, 2, 4])
 @pytest.mark.parametrize("n,k,g,dtype", [(4096, 12288, 128, "bf16"), (520, 10240, 128, "bf16"),
                                          (264, 16384, 256, "fp16"), (100, 12288, 128, "fp16")])
-def test_decode_long_k(m, n, k, g, dtype):
+def test_decode_long_k(m, n, k, g, dtype, with_and_without_rows):
     """M <= 4 at long K (80-128 K tiles, more than the round-robin kernel's one load batch
-    holds): the split-K decode kernel, with 128- and 256-wide groups, fp16 x and ragged N."""
+    holds): the rows kernel and the split-K decode kernel, with 128- and 256-wide groups, fp16 x and
+    ragged N."""
     packed, s = int4_case(n, k, g, 1, seed=n + k + m)
     w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), scale_tensor(s), 1, g)
     x = x_case(m, k, dtype, seed=m + 3)
@@ -467,8 +470,8 @@ def _edge_scales(n, groups, seed):
 
 @pytest.mark.parametrize("m", [1, 16, 256])
 @pytest.mark.parametrize("sdt", ["fp32", "bf16"])
-def test_int4_scale_domain_edge_exact(m, sdt):
-    """Scales just below 2^120 (where (128 + q + 8) s still fits fp32) go through the decode
+def test_int4_scale_domain_edge_exact(m, sdt, with_and_without_rows):
+    """Scales just below 2^120 (where (128 + q + 8) s still fits fp32) go through the decode and rows
     (M = 1, 16) and MFMA (M = 256) kernels exactly: the identity rows of x pick out
     round(q round(s)) bit for bit, as test_marlin.cpp:54-78 does for ordinary scales."""
     n, k, g = 64, 256, 128
@@ -542,10 +545,10 @@ def test_int4_scale_check_from_several_threads():
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 4096, 6144), (4, 4096, 24576), (1, 12288, 512), (3, 12288, 512)])
-def test_int4_scales_across_ranges_exact(m, k, n):
+def test_int4_scales_across_ranges_exact(m, k, n, with_and_without_rows):
     """Scales mostly ordinary, with scattered groups below 2^-17 or at 2^16 and above, and one
     strip entirely at 2^-18, through the decode kernels (round-robin at K = 4096, split-K at
-    K = 12288): identity rows of x must pick out round(q round(s)) bit for bit in every
+    K = 12288) and the rows kernel: identity rows of x must pick out round(q round(s)) bit for bit in every
     column."""
     g = 128
     print(f"scale ranges m={m} k={k} n={n}", flush=True)

@@ -161,8 +161,8 @@ def test_mlp_block_quantized_matches_dense(kind, m):
     """A Qwen3-style MLP block (gate_up, silu·mul, down) through linear::int4 / linear::fp8
     and silu_mul_cuda, against the same block on the dequantized weights in fp32: the
     model-level comparison of test_qwen3_5.cpp:691-696 (fp8 in 32 x 32 blocks there), with its
-    bound, max |y - ref| / max |ref| < 5e-2. M = 1 and 16 run the decode kernels, 24 the
-    two-row-block decode kernels, 64 the MFMA kernel."""
+    bound, max |y - ref| / max |ref| < 5e-2. The 32-wide fp8 blocks run the decode kernels (M = 1, 16
+    and, with two row blocks, 24) and the MFMA kernel (64), the other formats the rows kernel too."""
     hidden, inter = 512, 1024
     g = gen(40 + m)
     w_gu = (torch.randn((2 * inter, hidden), generator=g, **cuda(torch.float)) * 0.02).to(torch.bfloat16)

@@ -1,7 +1,7 @@
 """plm_gemm_noalloc (no workspace, no allocation: a fixed device scratch array) against
 plm_gemm with a workspace, through the C ABI: bit for bit, on two calls in a row, the
-second with a smaller input, for int4 and fp8 shapes that split K on the decode kernel and
-on the MFMA kernel; its first call on the device made inside a HIP graph capture (fresh
+second with a smaller input, for int4 and fp8 shapes that split K on the rows, decode and
+MFMA kernels; its first call on the device made inside a HIP graph capture (fresh
 process) and the graph replayed; and a call needing more scratch than the fixed array is
 refused."""
 
@@ -56,15 +56,15 @@ def _with_workspace(x, w, sc, n, k, fmt="int4"):
 
 
 @pytest.mark.parametrize("case", [
-    # (format, n, k, first M, second M): decode kernel with a K split across workgroups
+    # (format, n, k, first M, second M): rows kernel, or decode kernel with a K split across workgroups
     ("int4", 4096, 12288, 16, 5),
     # MFMA kernel with a K split (fewer work tiles than CUs)
     ("int4", 4096, 4096, 256, 100),
-    # fp8 weights, 128 x 128 block scales: decode kernel with a K split, then the MFMA kernel
+    # fp8 weights, 128 x 128 block scales: the same, then the MFMA kernel
     ("fp8", 5120, 17408, 16, 7),
     ("fp8", 2048, 4096, 256, 64),
 ])
-def test_noalloc_matches_workspace_entry_point(case):
+def test_noalloc_matches_workspace_entry_point(case, with_and_without_rows):
     fmt, n, k, m1, m2 = case
     lib = _lib.load()
     assert 0 < lib.plm_gemm_workspace_bytes(_FMT[fmt][0], m1, n, k) <= (32 << 20)
@@ -122,7 +122,7 @@ _CAPTURE_SCRIPT = textwrap.dedent("""
 
 def test_noalloc_first_call_inside_graph_capture():
     lib = _lib.load()
-    assert lib.plm_gemm_workspace_bytes(_lib.PLM_INT4, 16, 4096, 12288) > 0  # the decode kernel splits K
+    assert lib.plm_gemm_workspace_bytes(_lib.PLM_INT4, 16, 4096, 12288) > 0  # a plan that splits K
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     print("noalloc first call under capture (subprocess)", flush=True)
     res = subprocess.run([sys.executable, "-c", _CAPTURE_SCRIPT.format(root=root)], capture_output=True, text=True,
