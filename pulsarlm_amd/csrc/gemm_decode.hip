@@ -1003,9 +1003,6 @@ rr_config choose_rr(int64_t m, int64_t n, int64_t k, plm_format f, bool a8) {
     return c;
 }
 
-// x rows are staged in LDS for M up to this (above it the 16-byte loads of x are mostly full).
-constexpr int64_t kStageMaxM = 4;
-constexpr int64_t kStageMaxBytes = 96 * 1024;  // staging area per workgroup
 bool no_x_staging() { return knobs().decode_no_xs; }  // A/B measurements
 
 // The round-robin kernel's LDS layout for a call, and whether it takes the call.

@@ -130,46 +130,67 @@ static int64_t rows_need(const rows_plan& p) {
 }
 int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k) { return rows_need(plan_rows(f, m, n, k)); }
 
-// The rows kernel or the decode / MFMA kernels, by both sides' times at the layers above and at 31
-// random ones (hidden 2048..5120, M = 1..128; us, without -> with the rows kernel). rr: the
-// round-robin decode kernel takes the call.
-// * 17 to 64 rows: the rows kernel (against the MFMA kernel int4 1.1-2.0x, fp8 1.01-1.8x), but int4
-//   above 32 rows with more than four strips per CU, where the MFMA kernel is even or faster (K 4736,
-//   N 21248, M = 64: 28.6 -> 32.7) unless three-strip tiles nearly fill whole rounds of the CUs and there
-//   are at most 48 rows (K 5120, N 23040: M = 36 31.0 -> 29.3, M = 48 30.5 -> 30.7).
-// * Above 64 the weights are read once per row block: up to two strips per CU and K = 8448 (int4
-//   K 4736, N 5248, M = 96: 19.4 -> 15.0, K 8192, N 2432, M = 128: 16.2 -> 15.4; fp8 K 2944, N 3968, M = 128:
-//   18.8 -> 11.0; beyond: int4 K 2048, N 8704, M = 96 14.3 -> 15.2, K 9088, N 3200, M = 112 21.8 -> 24.8).
-// * Up to 16 rows int4: the round-robin kernel where it applies (3-8 % faster), but above 4 rows
-//   with five strips or more per CU (K 4096, N 24576, M = 16: 15.4 -> 14.6). Elsewhere (long K,
-//   groups below 128) the rows kernel (K 14336, N 5120, M = 1: 14.9 -> 12.3; K 8192, N 8192: 12.3 -> 9.6), but
-//   up to 4 rows exactly one strip per CU over a K that the split-K decode kernel holds in three
-//   load batches a wavefront (K 12288, N 4096: 8.1 against 9.3 at best; K 13312: 11.6 -> 9.7), and up
-//   to 2 rows groups below 128 with four strips or more per CU (K 4992, N 24832: 25.9 -> 28.5).
-// * Up to 16 rows fp8: the rows kernel, but the round-robin one with four strips or more per CU
-//   up to 4 rows (K 3968, N 25600: 19.2 -> 23.4) and the split-K one up to 2 rows where that one does
-//   not apply (K 4864, N 32768: 28.7 -> 30.6); and between one and 1.5 strips per CU, or up to one
-//   above 4 rows, up to K = 5120 (even to 9 % slower); and up to 2 rows the split-K one at long K and
-//   at most one strip per CU (K 12800, N 3968: 12.6 -> 13.7).
+// The rows kernel or the decode / MFMA kernels, by both sides' times at 1120 random layers (N = 128..40000,
+// K = 256..28672, groups of 16 to 640 and every scale type) and 20 to 25 row counts each. What decides is
+// how many strips a CU gets and how many K tiles there are: the rows kernel's start and epilogue are paid
+// per round of its workgroups (one to four strips each), and below 16 K tiles its eight wavefronts have less than
+// two each. Ratios below are rows / other kernel, means over the layers of a range. rr: the round-robin
+// decode kernel takes the call.
 bool use_rows(plm_format f, int64_t m, int64_t n, int64_t k, int64_t group_size, bool rr) {
     const tuning& t = knobs();
     if (t.rows_force) return true;
     if (t.rows_off || t.decode_max_m >= 0 || t.decode_sp > 0 || t.rr_sg > 0 || t.decode_no_xs || t.mfma_shape) return false;
-    const int64_t strips = ceil_div(n, kTileN), cus = cu_count();
-    const bool sub = group_size % kTileK != 0;
-    if (m > 64) return strips <= 2 * cus && k <= 66 * kTileK;
-    if (m > 16) {
-        const int64_t tiles3 = ceil_div(strips, 3);
-        return f == PLM_FP8 || m <= 32 || strips <= 4 * cus || (m <= 48 && 10 * tiles3 >= 9 * round_up(tiles3, cus));
+    const int64_t strips = ceil_div(n, kTileN), kt = ceil_div(k, kTileK), cus = cu_count();
+    const bool sub = group_size % kTileK != 0, fp8 = f == PLM_FP8;
+    auto up_to = [&](int64_t per_cu) { return strips <= per_cu * cus; };
+    // Against the MFMA kernel. Above 64 rows the weights are read once per row block: up to one strip
+    // per CU 0.35-0.95, up to two 0.5-0.9 but 1.0-1.2 past 64 K tiles, beyond 1.1-2.
+    if (m > 64) return up_to(1) || (up_to(2) && kt > 2 && kt <= 64);
+    if (m > 32) {
+        if (up_to(4)) {  // 0.4-0.95
+            if (kt <= (fp8 ? 4 : 8)) return up_to(kt > 2 ? 3 : 2);  // past it 1.0-1.15
+            return fp8 || m <= 48 || kt <= 64 || up_to(2) || !up_to(3);  // int4 else 1.04-1.2
+        }
+        if (m > 48) return false;  // 1.0-1.8
+        if (fp8) return kt > 8 && kt <= 64;  // 0.83-0.99; below 1.0-1.3, above 1.0-1.15
+        return !up_to(5) && (up_to(6) ? kt >= 16 && kt <= 32 : kt >= 24 && kt <= 64);  // 0.84-1.0; outside 1.0-1.5
     }
-    if (f == PLM_FP8) {
-        if (strips >= 4 * cus && m <= (rr ? 4 : 2)) return false;
-        if (strips <= cus) return m <= 4 ? rr || m > 2 : !(rr || k <= 5120);
-        return 2 * strips > 3 * cus || !(rr || k <= 5120);
+    // 17 to 32 rows: 0.5-0.95; with fewer K tiles and more strips 1.05-2 against the decode kernels,
+    // which stop at 24 rows from four strips per CU on.
+    if (m > 16) return kt > 16 || up_to(3) || (up_to(6) && kt > (m > 24 ? 4 : 8));
+    // Against the decode kernels. Where the round-robin one applies it is 3-25 % faster, but for int4 above
+    // 4 rows from five strips per CU on (0.7-1.0), and for fp8 (up to 4 rows 0.75-0.97, above 0.7-0.95 past
+    // 1.5 strips per CU) only between one and 1.5 strips per CU, and up to 4 rows from four on.
+    if (rr) {
+        if (!fp8) return m > 4 && strips >= 5 * cus;
+        return m <= 4 ? up_to(1) || (2 * strips > 3 * cus && strips < 4 * cus) : 2 * strips > 3 * cus;
     }
-    if (rr) return m > 4 && strips >= 5 * cus;
-    if (sub) return m > 2 || strips < 4 * cus;
-    return m > 4 || strips != cus || k > 12288;
+    // Against the split-K one.
+    if (fp8) {
+        if (kt <= 4) return false;  // 1.0-1.4
+        if (kt <= 8) return up_to(1) || (m > 4 && up_to(2));  // 0.7-0.8; past it 1.05-1.3
+        if (up_to(1)) return m > 4 || 2 * strips <= cus || kt <= 32 || kt > 96;  // 0.63-0.98; else 1.0-1.17
+        if (2 * strips <= 3 * cus) return m > 4 || kt <= 16 || kt > (m > 2 ? 64 : 96);  // 0.64-0.97; else 1.0-1.15
+        if (m <= 2) return m == 2 && kt > 96 && strips < 4 * cus;  // 0.88-0.91; else 1.0-1.2
+        if (kt <= 16) return m > 4 && up_to(3);  // 0.65-0.98; past it 1.0-1.25
+        if (kt <= 32) return m <= 4 ? up_to(2) : up_to(3) || (m > 8 && kt > 24);  // 0.8-0.99; past it 1.0-1.15
+        return m <= 4 || m > 8 || up_to(4) || kt > 48;  // 0.75-0.99; past it 1.0-1.1
+    }
+    if (kt <= 4) return m > 4 && up_to(sub ? 6 : 1);  // 0.8-1.0; past it 1.05-1.4
+    if (kt <= 8) return up_to(1) || (m > 4 && (up_to(3) || sub));  // 0.55-0.98; past it 1.0-1.3
+    // Exactly one strip per CU over a K whose x the split-K kernel holds in LDS: it runs unsplit in one
+    // round (K 13312, M = 1: 8.6 us against 9.5; K 20480, M = 2: 11.6 against 13.0). With fewer strips it
+    // splits K, with more it takes a second round (K 13312, M = 1, N 4080: 12.1 against 9.8, N 4112: 13.7
+    // against 11.2), and x from global memory costs it the lead (K 13312, M = 4: 11.5 against 9.7).
+    if (!sub && strips == cus && m * k * 2 <= kStageMaxBytes && m <= kStageMaxM) return false;
+    // 0.4-0.98, but groups of whole tiles at 17 to 32 K tiles 1.03-1.07 up to 2 rows.
+    if (up_to(4)) return m > 2 || sub || kt <= 16 || kt > 32 || 2 * strips <= 3 * cus;
+    // Past four strips per CU the split-K kernel takes two strips a wavefront: up to 2 rows 0.8-0.95 (N 18944,
+    // K 4480, M = 1: 13.3 us against 13.7; K 6144: 16.2 against 17.1), up to 4 (x of 3 rows and more
+    // costs it a quarter past 32 K tiles) and 8 rows 0.85-0.97 against the rows kernel outside these.
+    if (m <= 2) return sub ? kt <= 16 || kt > 48 : kt > (m == 1 ? 96 : 64);
+    if (m <= 4) return kt > 32 || (sub && kt <= 16);
+    return sub || m > 8 || kt > 48;
 }
 
 // A call as the rows kernel would run it; `taken` is false where it does not take the call (the

@@ -282,6 +282,10 @@ constexpr int kOOB = 0x40000000;
 // launch_decode with the fused W8A8 quantizer requested, when its kernel does not apply to
 // the shape (the caller then quantizes in a launch of its own). Not a plm_status value.
 constexpr int kDecodeNotTaken = -1;
+// The split-K decode kernel stages x rows in LDS for M up to this (above it the 16-byte loads of x are
+// mostly full).
+constexpr int64_t kStageMaxM = 4;
+constexpr int64_t kStageMaxBytes = 96 * 1024;  // staging area per workgroup
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0), static_cast<int>(bytes),
                                              0x00020000);
