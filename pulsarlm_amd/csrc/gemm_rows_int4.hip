@@ -128,9 +128,7 @@ static int64_t rows_need(const rows_plan& p) {
     if (p.rb == 0 || p.splits <= 1) return 0;
     return kCounterBytes + static_cast<int64_t>(p.m_blocks) * p.n_blocks * p.splits * p.rb * p.sg * 1024;
 }
-int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k) { return rows_need(plan_rows(f, m, n, k)); }
-
-// The rows kernel or the decode / MFMA kernels, by both sides' times at 1120 random layers (N = 128..40000,
+// The rows kernel or the decode / MFMA kernels, by both sides' times at 1358 random layers (N = 128..40000,
 // K = 256..28672, groups of 16 to 640 and every scale type) and 20 to 25 row counts each. What decides is
 // how many strips a CU gets and how many K tiles there are: the rows kernel's start and epilogue are paid
 // per round of its workgroups (one to four strips each), and below 16 K tiles its eight wavefronts have less than
@@ -191,6 +189,14 @@ bool use_rows(plm_format f, int64_t m, int64_t n, int64_t k, int64_t group_size,
     if (m <= 2) return sub ? kt <= 16 || kt > 48 : kt > (m == 1 ? 96 : 64);
     if (m <= 4) return kt > 32 || (sub && kt <= 16);
     return sub || m > 8 || kt > 48;
+}
+
+// For calls of a size: no group size or scale layout, so what any of them may need.
+int64_t rows_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k) {
+    if (m > kRowsMaxM) return 0;
+    const bool any = use_rows(f, m, n, k, kTileK, false) || use_rows(f, m, n, k, kTileK, true) ||
+                     (f == PLM_INT4 && use_rows(f, m, n, k, kTileK / 2, false));
+    return any ? rows_need(plan_rows(f, m, n, k)) : 0;
 }
 
 // A call as the rows kernel would run it; `taken` is false where it does not take the call (the

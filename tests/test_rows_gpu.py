@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from pulsarlm_amd import ops
+from pulsarlm_amd import _lib, ops
 from tests._util import TDT, assert_close, force_rows, fp8_case, int4_case, rows_plan, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
@@ -130,23 +130,29 @@ def test_split_rows_graph_replays_match_eager(fmt, m, n, k):
         assert torch.equal(run(), eager), f"eager after replay {i}"
 
 
-def test_small_workspace_keeps_the_general_path():
-    """A workspace that only the decode / MFMA kernels' needs fit is still accepted, with their result."""
-    from pulsarlm_amd import _lib
-
+@pytest.mark.parametrize("m,n,k", [(24, 4096, 12288), (5, 4096, 12288)])
+def test_small_workspace_keeps_the_general_path(m, n, k, tuning_env):
+    """A workspace that only the decode kernels' need fits is accepted, with their result to the bit; one
+    below that is refused."""
     lib = _lib.load()
-    m, n, k = 48, 4096, 4096
     packed, s, (w, sc) = _int4(n, k, 128, "fp16", seed=8)
     x = to_dev(x_case(m, k, "bf16", seed=8), torch.bfloat16)
     full = lib.plm_gemm_workspace_bytes(_lib.PLM_INT4, m, n, k)
-    want = ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128).float()
-    for nbytes in (full, full - 1, 0):
+    by_rows = ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128)
+    p = rows_plan("int4", m, n, k, 1, 128, "fp16")
+    assert full == 65536 + p["m_blocks"] * p["n_blocks"] * p["splits"] * p["rb"] * p["sg"] * 1024
+    tuning_env("PLM_ROWS", "0")
+    general = lib.plm_gemm_workspace_bytes(_lib.PLM_INT4, m, n, k)
+    by_decode = ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128)
+    tuning_env("PLM_ROWS", None)
+    assert 0 < general < full and not torch.equal(by_rows, by_decode)
+    for nbytes, want in ((full, by_rows), (full - 1, by_decode), (general, by_decode), (general - 1, None), (0, None)):
         ws = torch.zeros(max(nbytes, 1), dtype=torch.uint8, device="cuda")
         y = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
         rc = lib.plm_gemm(_lib.PLM_INT4, x.data_ptr(), _lib.PLM_BF16, w.data_ptr(), sc.data_ptr(), _lib.PLM_FP16, m, n, k, 1,
                           128, y.data_ptr(), ws.data_ptr() if nbytes else None, nbytes,
                           torch.cuda.current_stream().cuda_stream)
-        if rc == _lib.PLM_OK:
-            assert torch.allclose(y.float(), want, rtol=2e-2, atol=2e-2), nbytes
+        if want is None:
+            assert rc == _lib.PLM_ERR_WORKSPACE, nbytes
         else:
-            assert rc == _lib.PLM_ERR_WORKSPACE and nbytes < full
+            assert rc == _lib.PLM_OK and torch.equal(y, want), nbytes

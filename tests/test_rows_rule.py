@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import pytest
 
+from pulsarlm_amd import _lib
 from tests._util import rows_plan
 
 
@@ -28,3 +29,13 @@ from tests._util import rows_plan
 def test_rows_rule(fmt, m, n, k, g, rows):
     plan = rows_plan(fmt, m, n, k, 1 if fmt == "int4" else 128, g, "fp16" if fmt == "int4" else "fp32")
     assert (plan is not None) == rows
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("fp8", 2, 5290, 8576), ("int4", 2, 17026, 4864), ("fp8", 4, 4850, 5088)])
+def test_no_workspace_for_a_kernel_that_no_call_of_the_size_takes(fmt, m, n, k, tuning_env):
+    """The size query counts the rows kernel's K split only where some group size takes the call there."""
+    f = _lib.PLM_INT4 if fmt == "int4" else _lib.PLM_FP8
+    assert all(rows_plan(fmt, m, n, k, 1, g, "fp32") is None for g in (16, 128, 256))
+    assert _lib.load().plm_gemm_workspace_bytes(f, m, n, k) == 0
+    tuning_env("PLM_ROWS", "1")
+    assert _lib.load().plm_gemm_workspace_bytes(f, m, n, k) > 0
