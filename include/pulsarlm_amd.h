@@ -107,7 +107,9 @@ int plm_dequant(plm_format format, const void* weight, const void* scale, plm_dt
                 int64_t n, int64_t k, int64_t block_n, int64_t group_size,
                 void* out, plm_dtype out_dtype, void* stream);
 
-/* Workspace bytes plm_gemm may use for an [M, K] x [N, K]^T call (0 if none). */
+/* Workspace bytes plm_gemm may use for an [M, K] x [N, K]^T call (0 if none). A call that is given
+ * fewer either fails with PLM_ERR_WORKSPACE or runs with K split another way: its sums are then
+ * taken in another order. For one workspace size the results are the same bits on every call. */
 int64_t plm_gemm_workspace_bytes(plm_format format, int64_t m, int64_t n, int64_t k);
 
 /*

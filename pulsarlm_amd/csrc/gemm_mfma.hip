@@ -185,22 +185,20 @@ int64_t mfma_contract_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool 
 }
 
 namespace {
-struct mfma_plan {
-    mfma_config config;  // with any workspace
-    int64_t contract;
-};
-const mfma_plan& plan_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8) {
-    thread_local plan_cache<mfma_plan> cache;
-    return cache.get(f + (a8 ? 2 : 0), m, n, k,
-                     [&] { return mfma_plan{choose_mfma(f, m, n, k, a8, INT64_MAX), mfma_contract_bytes(f, m, n, k, a8)}; });
+// The plan within `limit` workspace bytes, and with any.
+mfma_config plan_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, int64_t limit = INT64_MAX) {
+    thread_local plan_cache<mfma_config> cache;
+    return cache.get(f + (a8 ? 2 : 0), m, n, k, limit, [&] { return choose_mfma(f, m, n, k, a8, limit); });
 }
 }  // namespace
 
-int64_t mfma_contract(plm_format f, int64_t m, int64_t n, int64_t k, bool a8) { return plan_mfma(f, m, n, k, a8).contract; }
+int64_t mfma_contract(plm_format f, int64_t m, int64_t n, int64_t k, bool a8) {
+    thread_local plan_cache<int64_t> cache;
+    return cache.get(f + (a8 ? 2 : 0), m, n, k, 0, [&] { return mfma_contract_bytes(f, m, n, k, a8); });
+}
 
 int64_t mfma_workspace_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool a8) {
-    const mfma_plan& p = plan_mfma(f, m, n, k, a8);
-    return std::max(p.contract, p.config.need);
+    return std::max(mfma_contract(f, m, n, k, a8), plan_mfma(f, m, n, k, a8).need);
 }
 
 namespace {
@@ -224,14 +222,14 @@ int launch_mfma(const char* op, plm_format f, const void* x, bool bf16, const vo
                 void* workspace, size_t workspace_bytes, hipStream_t s, const uint8_t* xq, const float* x_scale) {
     PLM_CHECK_ARG(k <= (int64_t{1} << 21), op, "K above 2^21 is not supported");
     const bool a8 = xq != nullptr;
-    const mfma_plan plan = plan_mfma(f, m, n, k, a8);
-    const int64_t need = plan.contract;
+    const int64_t need = mfma_contract(f, m, n, k, a8);
     if (need > 0 && (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need)) {
         set_error(op, "workspace of %lld bytes required, %zu given", static_cast<long long>(need), workspace_bytes);
         return PLM_ERR_WORKSPACE;
     }
     const int64_t have = workspace != nullptr ? static_cast<int64_t>(workspace_bytes) : 0;
-    const mfma_config c = plan.config.need <= have ? plan.config : choose_mfma(f, m, n, k, a8, have);
+    mfma_config c = plan_mfma(f, m, n, k, a8);
+    if (c.need > have) c = plan_mfma(f, m, n, k, a8, have);
     mfma_args a{};
     fill_common(a, x, w, scale, scale_dtype, m, n, k, block_n, group_size, y);
     a.splits = c.splits;

@@ -121,7 +121,7 @@ rows_plan make_rows_plan(plm_format f, int64_t m, int64_t n, int64_t k) {
 rows_plan plan_rows(plm_format f, int64_t m, int64_t n, int64_t k) {
     if (m < 1 || m > kRowsMaxM || k > kRowsMaxK || n > (int64_t{1} << 24)) return rows_plan{};
     thread_local plan_cache<rows_plan> cache;
-    return cache.get(f, m, n, k, [&] { return make_rows_plan(f, m, n, k); });
+    return cache.get(f, m, n, k, 0, [&] { return make_rows_plan(f, m, n, k); });
 }
 
 static int64_t rows_need(const rows_plan& p) {

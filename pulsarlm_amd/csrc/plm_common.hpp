@@ -466,24 +466,25 @@ struct tuning {
 };
 const tuning& knobs();
 
-// The plans of the last sizes a thread has called with (a pure function of the sizes and the
-// knobs; working one out takes a few us, as long as a short kernel): 64 entries per thread.
+// The plans of the last sizes a thread has called with (a pure function of the sizes, the bytes it
+// may use and the knobs; working one out takes a few us, as long as a short kernel): 64 entries per thread.
 template <typename P> struct plan_cache {
     struct entry {
-        int64_t m = -1, n = 0, k = 0;
+        int64_t m = -1, n = 0, k = 0, limit = 0;
         int kind = 0;
         unsigned epoch = 0;
         P plan{};
     };
     entry entries[64];
-    template <typename Fn> const P& get(int kind, int64_t m, int64_t n, int64_t k, Fn make) {
+    template <typename Fn> const P& get(int kind, int64_t m, int64_t n, int64_t k, int64_t limit, Fn make) {
         const uint64_t h = (static_cast<uint64_t>(m) * 0x9E3779B97F4A7C15u) ^ (static_cast<uint64_t>(n) * 0xC2B2AE3D27D4EB4Fu) ^
-                           (static_cast<uint64_t>(k) * 0x165667B19E3779F9u) ^ static_cast<uint64_t>(kind);
+                           (static_cast<uint64_t>(k) * 0x165667B19E3779F9u) ^ (static_cast<uint64_t>(limit) * 0x27D4EB2F165667C5u) ^
+                           static_cast<uint64_t>(kind);
         entry& e = entries[(h ^ (h >> 29)) >> 7 & 63];
         const unsigned epoch = knobs().epoch;
-        if (e.m != m || e.n != n || e.k != k || e.kind != kind || e.epoch != epoch) {
+        if (e.m != m || e.n != n || e.k != k || e.limit != limit || e.kind != kind || e.epoch != epoch) {
             e.plan = make();
-            e.m = m, e.n = n, e.k = k, e.kind = kind, e.epoch = epoch;
+            e.m = m, e.n = n, e.k = k, e.limit = limit, e.kind = kind, e.epoch = epoch;
         }
         return e.plan;
     }

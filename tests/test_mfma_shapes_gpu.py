@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from pulsarlm_amd import ops
+from pulsarlm_amd import _lib, ops
 from tests._util import TDT, assert_close, force_mfma, fp8_case, int4_case, mfma_plan, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
@@ -109,3 +109,37 @@ def test_xcd_patches(m, n, shape, splits, tuning_env):
         assert p["tile"] == (256, 256) and p["halves"], p
     y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
     assert_close(ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128, out=y), to_np(x.double() @ dense.t()), f"{shape} {m}x{n}")
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("int4", 333, 4096, 4096), ("fp8", 300, 1024, 4096)])
+def test_plan_follows_the_workspace(fmt, m, n, k):
+    """Calls of one size with several workspaces in turn, from what the plan asks for down to what is
+    refused: each is within tolerance, a smaller one splits K otherwise, and each size of workspace gives
+    its own bits every time (plans are kept by the bytes they may use)."""
+    lib = _lib.load()
+    rng = np.random.default_rng(4)
+    x = to_dev(x_case(m, k, "bf16", seed=4), torch.bfloat16)
+    if fmt == "int4":
+        packed, s = int4_case(n, k, 128, 1, seed=4)
+        w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), to_dev(s), 1, 128)
+        f, bn, sdt = _lib.PLM_INT4, 1, _lib.PLM_FP16
+    else:
+        codes, scale = O.fp8_block_quantize(O.bf16_round(rng.standard_normal((n, k)).astype(np.float32) * 0.02), 128, 128)
+        w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), to_dev(scale), 128, 128)
+        f, bn, sdt = _lib.PLM_FP8, 128, _lib.PLM_FP32
+    ref = to_np(x.double() @ ops.dequant_marlin_cuda(fmt, w, sc, n, k, bn, 128).double().t())
+    full = lib.plm_gemm_workspace_bytes(f, m, n, k)
+    sizes, seen = [full, full - 1, 3 * full // 4, full // 2 + 65536], {}
+    ws = torch.zeros(full, dtype=torch.uint8, device="cuda")
+    for i in range(3):
+        for nbytes in sizes:
+            y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            rc = lib.plm_gemm(f, x.data_ptr(), _lib.PLM_BF16, w.data_ptr(), sc.data_ptr(), sdt, m, n, k, bn, 128, y.data_ptr(),
+                              ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+            if rc == _lib.PLM_ERR_WORKSPACE:
+                assert nbytes < full - 1
+                continue
+            assert rc == _lib.PLM_OK
+            assert_close(y, ref, f"{nbytes} of {full} bytes, call {i}")
+            assert torch.equal(seen.setdefault(nbytes, y), y), f"{nbytes} of {full} bytes, call {i}"
+    assert any(not torch.equal(y, seen[full]) for y in seen.values())
