@@ -70,10 +70,14 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
         const shape sh = kShapeOf[id];
         const shape_cost& sc = mc.shapes[id];
         const int64_t m_blocks = ceil_div(m, sh.bm()), n_blocks = ceil_div(strips, sh.bs()), tiles = m_blocks * n_blocks;
-        const int slots = sc.step[2] > 0 ? 3 : (sc.step[1] > 0 ? 2 : 1);
         const double tile_mib = sh.bm() * sh.bs() * kTileN * 4.0 / (1 << 20);
-        const double memory = static_cast<double>(tiles * ktiles) * (sh.bm() * (a8 ? 128 : 256) + sh.bs() * tile_bytes(f)) / 1e6 * mc.memory;
-        auto loop = [&](int64_t wgs, double tps) {  // `wgs` workgroups of tps K tiles over the CUs
+        // us to bring in `of` tiles of the call's K: x rows and strips.
+        auto memory = [&](int64_t of, int rows) {
+            return static_cast<double>(of * ktiles) * (rows * (a8 ? 128 : 256) + sh.bs() * tile_bytes(f)) / 1e6 * mc.memory;
+        };
+        // `wgs` workgroups of tps K tiles over the CUs, no faster than `floor`.
+        auto loop = [&](const shape_cost& sc, int64_t wgs, double tps, double floor) {
+            const int slots = sc.step[2] > 0 ? 3 : (sc.step[1] > 0 ? 2 : 1);
             const double per_cu = wgs <= 4 * cus ? static_cast<double>(ceil_div(wgs, cus))
                                                  : static_cast<double>(wgs) / static_cast<double>(cus) + 0.5;
             const int whole = static_cast<int>(per_cu / slots);
@@ -81,7 +85,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
             const int lo = static_cast<int>(rest);
             double g = whole * sc.step[slots - 1];
             if (rest > 0) g += lo + 1 > slots ? 0.0 : (lo > 0 ? sc.step[lo - 1] : 0.0) + (rest - lo) * (sc.step[lo] - (lo > 0 ? sc.step[lo - 1] : 0.0));
-            const double steps = (tps + sc.fill) * g, x = steps * steps * steps, y = memory * memory * memory;
+            const double steps = (tps + sc.fill) * g, x = steps * steps * steps, y = floor * floor * floor;
             return std::cbrt(std::sqrt(x * x + y * y));  // the larger one, rounded where they meet
         };
         for (int64_t want = 1; want <= std::min<int64_t>(8, ktiles); ++want) {
@@ -92,21 +96,27 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
             c.shape = id;
             c.m_blocks = static_cast<int>(m_blocks), c.n_blocks = static_cast<int>(n_blocks);
             c.splits = static_cast<int>(splits), c.tiles_per_split = static_cast<int>(tps);
-            double cost = mc.launch + loop(tiles * splits, static_cast<double>(tps));
+            double cost = mc.launch + loop(sc, tiles * splits, static_cast<double>(tps), memory(tiles, sh.bm()));
             if (splits > 1) {
                 const int64_t partials = tiles * splits * sh.bm() * sh.bs() * kTileN * 4;
                 c.need = kCounterBytes + partials;
                 if (partials > kMfmaMaxPartials || c.need > limit) break;
                 cost += mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(tiles * splits);
             }
+            // A tail launch: whole rounds, then the rest as halves or with K split. Each launch brings in its
+            // own share of the tiles, and a tail's steps take longer than a whole call's: 1.15 times for
+            // halves; 1.1 times for a K split, and 4 us and 1.5 us for each tile that the last workgroup
+            // adds up. The pick is then 0.5-0.6 % (K split) and 0.6-0.8 % (halves) slower than the faster side, at
+            // about 340 sizes where a tail can be had and comes near; 2.5-5.5 % without tails. fp8 K 5120, N 34816,
+            // M = 2048 762 -> 676 us, K 17408, N 5120, M = 4096 738 -> 650; W8A8 K 5120, N 34816, M = 2048
+            // 406 -> 391; int4 the same size 664 -> 616.
             const int64_t rem = tiles % cus;
             if (id == kIdX && splits == 1 && tiles > cus && rem > 0 && 2 * rem <= cus && ktiles >= 8 && !t.mfma_no_tail &&
                 !t.mfma_unsplit && t.mfma_splits == 0) {
-                const double whole = mc.launch + loop(tiles - rem, static_cast<double>(tps));
+                const double whole = mc.launch + loop(sc, tiles - rem, static_cast<double>(tps), memory(tiles - rem, sh.bm()));
                 if (mode != kModeFp8 && rem % m_blocks == 0 && !t.mfma_no_halves) {
-                    // Halves: half-area tiles, assumed 10 % less efficient. (fp8 W8A16, whose tall
-                    // shape keeps the weights in registers, measured slower.)
-                    const double both = whole + 0.55 * loop(cus, static_cast<double>(tps));
+                    // (fp8 W8A16, whose tall shape keeps the weights in registers, measured slower with halves.)
+                    const double both = whole + 1.15 * loop(mc.shapes[kIdH], cus, static_cast<double>(tps), memory(2 * rem, kTallHalf.bm()));
                     if (both < cost) {
                         cost = both;
                         c.tail_tiles = static_cast<int>(rem), c.tail_halves = true;
@@ -116,8 +126,9 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
                     const int64_t ts = std::min<int64_t>(std::min<int64_t>(cus / rem, ktiles / 4), 8);
                     const int64_t ttps = ceil_div(ktiles, std::max<int64_t>(ts, 1)), tsp = ceil_div(ktiles, ttps);
                     const int64_t partials = rem * tsp * sh.bm() * sh.bs() * kTileN * 4;
-                    const double both = whole + mc.launch + loop(cus, static_cast<double>(ttps)) + mc.reduce +
-                                        mc.reduce_mib * tile_mib * static_cast<double>(rem * tsp);
+                    const double steps = loop(sc, cus, static_cast<double>(ttps), memory(rem, sh.bm()));
+                    const double exchange = mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(rem * tsp);
+                    const double both = whole + 1.1 * (steps + exchange) + 4.0 + 1.5 * static_cast<double>(tsp);
                     if (tsp >= 2 && rem <= kMaxCounters && kCounterBytes + partials <= limit && both < cost) {
                         cost = both;
                         c.tail_tiles = static_cast<int>(rem);

@@ -9,7 +9,7 @@ import torch
 
 from oracle import oracle as O
 from pulsarlm_amd import ops
-from tests._util import TDT, assert_close, fp8_case, to_dev, to_np
+from tests._util import TDT, assert_close, fp8_case, mfma_plan, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -97,6 +97,8 @@ def test_w8a8_full_size_tall_tail():
     scale, e4m3 weights times their 128x128 block scale. The products are exact, so the
     only differences are fp32 summation order and the bf16 output rounding."""
     m, k, n = 2048, 5120, 34816
+    plan = mfma_plan("w8a8", m, n, k)
+    assert plan["tile"] == (256, 256) and plan["tail"] == 64 and plan["halves"], plan
     g = torch.Generator(device="cpu").manual_seed(91)
     codes = torch.randint(0, 256, (n, k), generator=g, dtype=torch.int32).to(torch.uint8)
     codes[(codes == 0x7F) | (codes == 0xFF)] = 0  # no NaN codes
@@ -125,6 +127,9 @@ def test_config4_w8a16_m2048_every_row(shape):
     register-weight tiles with the K-split tail launch."""
     from tests.test_gemm_gpu import _check_full
     k, n = shape
+    if n == 34816:
+        plan = mfma_plan("fp8", 2048, n, k)
+        assert plan["tile"] == (256, 256) and plan["tail"] == 64 and plan["tail_splits"] > 1, plan
     g = torch.Generator(device="cpu").manual_seed(k + n)
     codes = torch.randint(0, 256, (n, k), generator=g, dtype=torch.int32).to(torch.uint8)
     codes[(codes == 0x7F) | (codes == 0xFF)] = 0

@@ -13,7 +13,7 @@ import torch
 
 from oracle import oracle as O
 from pulsarlm_amd import _lib, ops
-from tests._util import TDT, assert_close, force_mfma, fp8_case, int4_case, scale_tensor, to_dev, to_np, x_case
+from tests._util import TDT, assert_close, force_mfma, fp8_case, int4_case, mfma_plan, scale_tensor, to_dev, to_np, x_case
 
 pytestmark = pytest.mark.gpu
 
@@ -239,6 +239,9 @@ def test_gemm_graph_replays_match_eager(case, tuning_env):
     fmt, m, k, n = case[:4]
     tuning_env("PLM_ROWS", "0" if len(case) > 4 else None)
     print(f"graph replay case {case}", flush=True)
+    if m >= 2048:
+        plan = mfma_plan(fmt, m, n, k)
+        assert plan["tail"] and plan["halves"] == (fmt == "int4"), plan
     rng = np.random.default_rng(61)
     xd = torch.from_numpy(rng.standard_normal((m, k), dtype=np.float32)).to("cuda").to(torch.bfloat16)
     if fmt == "int4":
