@@ -131,11 +131,11 @@ int plm_gemm(plm_format format, const void* x, plm_dtype x_dtype,
  * forbid hipMalloc). No counterpart in the reference. The split-K partial sums and
  * arrival counters live in a fixed device array of PLM_NOALLOC_SCRATCH_BYTES inside the
  * library, one per GPU, held until the process ends; the first call on a device takes its
- * address and clears its counters (a kernel on `stream`). Calls needing more scratch than
- * that (plm_gemm_workspace_bytes) fail with PLM_ERR_INVALID. Every call on one GPU shares
+ * address and clears its counters (a kernel on `stream`). Calls that plm_gemm
+ * refuses with a workspace of that size fail with PLM_ERR_INVALID. Every call on one GPU shares
  * that GPU's array, so calls that may overlap on one GPU (different streams or threads)
- * race: use plm_gemm with separate workspaces for those. Same arguments and results as
- * plm_gemm otherwise.
+ * race: use plm_gemm with separate workspaces for those. Same arguments otherwise, and the results
+ * of plm_gemm with a workspace of that size.
  */
 #define PLM_NOALLOC_SCRATCH_BYTES (32 * 1024 * 1024)
 int plm_gemm_noalloc(plm_format format, const void* x, plm_dtype x_dtype,

@@ -81,6 +81,12 @@ int zero_output(const char* op, void* y, int64_t m, int64_t n, hipStream_t s) {
     return PLM_OK;
 }
 
+// Workspace bytes a plain call must bring; with more its plan may split K further.
+int64_t required_bytes(plm_format f, int64_t m, int64_t n, int64_t k) {
+    if (k == 0) return 0;
+    return use_decode(m, n) ? decode_workspace_bytes(f, m, n, k) : mfma_contract(f, m, n, k, false);
+}
+
 // Checked arguments to a kernel: the rows kernel where its rule takes the call, else the decode
 // or MFMA kernels. A call is refused for its workspace by those two paths' needs alone: one
 // that is too small for the rows kernel's K split only keeps the call from it.
@@ -89,7 +95,7 @@ int run_gemm(const char* op, plm_format f, const void* x, bool bf16, const void*
              size_t workspace_bytes, hipStream_t s) {
     if (k == 0) return zero_output(op, y, m, n, s);
     const bool decode = use_decode(m, n);
-    const int64_t need = decode ? decode_workspace_bytes(f, m, n, k) : mfma_contract(f, m, n, k, false);
+    const int64_t need = required_bytes(f, m, n, k);
     const bool enough = need == 0 || (workspace != nullptr && static_cast<int64_t>(workspace_bytes) >= need);
     if (enough && launch_rows(f, x, bf16, w, scale, scale_dtype, m, n, k, block_n, group_size, y, workspace, workspace_bytes, s)) {
         PLM_HIP_LAUNCH_CHECK(op);
@@ -275,7 +281,7 @@ int plm_gemm_noalloc(plm_format format, const void* x, plm_dtype x_dtype, const 
     if (int rc = check_gemm(op, format, x, x_dtype, weight, scale, scale_dtype, m, n, k, block_n, group_size, y))
         return rc;
     if (m == 0 || n == 0) return PLM_OK;
-    const int64_t need = plm_gemm_workspace_bytes(format, m, n, k);
+    const int64_t need = required_bytes(format, m, n, k);
     PLM_CHECK_ARG(need <= kScratchBytes, op,
                   "this call needs %lld bytes of split-K scratch, above the fixed %lld of plm_gemm_noalloc "
                   "(use plm_gemm with a workspace)",

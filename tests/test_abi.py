@@ -101,6 +101,34 @@ def test_zero_k_reaches_the_launch():
     assert res.returncode == 0 and "REACHED" in res.stdout, res.stdout + res.stderr
 
 
+def test_noalloc_takes_what_plm_gemm_takes_with_its_scratch():
+    """plm_gemm_noalloc refuses a call where plm_gemm does with a workspace of the fixed scratch's size, and
+    no other (a plan that would like more is planned within it): the calls get as far as their launch,
+    which has no device here."""
+    script = textwrap.dedent("""
+        import ctypes
+        from pulsarlm_amd import _lib
+        lib, d, scratch = _lib.load(), ctypes.c_void_p(256), 32 << 20
+        wanting = refused = 0
+        for fmt in (_lib.PLM_INT4, _lib.PLM_FP8):
+            for m in (1, 16, 40, 200, 433, 1024, 2048, 2508, 4175, 5341):
+                for n in (2048, 3455, 4096, 8327, 14166, 16958, 34816, 36895):
+                    for k in (128, 1792, 4096, 5120, 6144, 17408):
+                        a = (m, n, k, 1, 128, d)
+                        rc = lib.plm_gemm(fmt, d, _lib.PLM_BF16, d, d, _lib.PLM_FP32, *a, d, scratch, None)
+                        assert rc in (_lib.PLM_ERR_HIP, _lib.PLM_ERR_WORKSPACE), rc
+                        got = lib.plm_gemm_noalloc(fmt, d, _lib.PLM_BF16, d, d, _lib.PLM_FP32, *a, None)
+                        assert got == (_lib.PLM_ERR_HIP if rc == _lib.PLM_ERR_HIP else _lib.PLM_ERR_INVALID), (fmt, a)
+                        refused += rc != _lib.PLM_ERR_HIP
+                        wanting += rc == _lib.PLM_ERR_HIP and lib.plm_gemm_workspace_bytes(fmt, m, n, k) > scratch
+        assert wanting > 3 and refused > 20, (wanting, refused)
+        print("REACHED")
+    """)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")
+    res = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, cwd=HEADER.parents[1], env=env)
+    assert res.returncode == 0 and "REACHED" in res.stdout, res.stdout + res.stderr
+
+
 def test_repack_argument_errors():
     lib = _lib.load()
     d = ctypes.c_void_p(256)

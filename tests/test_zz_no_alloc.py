@@ -46,9 +46,10 @@ def _call(fn, x, w, sc, n, k, y, *tail, fmt="int4"):
     return rc
 
 
-def _with_workspace(x, w, sc, n, k, fmt="int4"):
+def _with_workspace(x, w, sc, n, k, fmt="int4", need=None):
     lib = _lib.load()
-    need = lib.plm_gemm_workspace_bytes(_FMT[fmt][0], x.shape[0], n, k)
+    if need is None:
+        need = lib.plm_gemm_workspace_bytes(_FMT[fmt][0], x.shape[0], n, k)
     ws = torch.zeros(max(need, 1), dtype=torch.uint8, device="cuda")
     y = torch.empty((x.shape[0], n), dtype=torch.bfloat16, device="cuda")
     _lib.check(_call("plm_gemm", x, w, sc, n, k, y, ws.data_ptr(), ws.numel(), fmt=fmt))
@@ -78,6 +79,19 @@ def test_noalloc_matches_workspace_entry_point(case, with_and_without_rows):
         ref = _with_workspace(x, w, sc, n, k, fmt=fmt)
         torch.cuda.synchronize()
         assert torch.equal(y, ref), f"M={m}"
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("int4", 2508, 14166, 1792), ("fp8", 2502, 7409, 4224)])
+def test_noalloc_plans_within_its_scratch(fmt, m, n, k):
+    """A call whose plan would like more than the fixed scratch, but that need not bring it: the bits of
+    plm_gemm with a workspace of that size."""
+    w, sc = (_weights if fmt == "int4" else _fp8_weights)(n, k, seed=m)
+    x = torch.randn(m, k, generator=torch.Generator("cuda").manual_seed(m), device="cuda").to(torch.bfloat16)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    _lib.check(_call("plm_gemm_noalloc", x, w, sc, n, k, y, fmt=fmt))
+    assert torch.equal(y, _with_workspace(x, w, sc, n, k, fmt=fmt, need=32 << 20))
+    ref = _with_workspace(x, w, sc, n, k, fmt=fmt).float()  # K split another way: two bf16 roundings apart
+    assert (y.float() - ref).norm() <= 2 * 2.0**-8 * ref.norm()
 
 
 # Run in a fresh process so that the first plm_gemm_noalloc call on the device (the scratch
