@@ -53,7 +53,10 @@ constexpr mode_cost kModeCost[3] = {
       {{0.9717, 0, 0}, 5.03}, {{0.7791, 1.0045, 0}, 2.87}, {{0.7998, 1.5840, 0}, 1.80}, {{0.6252, 0.8124, 0}, 3.44},
       {{0.6875, 0.8929, 0}, 3.56}, {}}}};
 
-constexpr int64_t kMfmaMaxPartials = 24 << 20;  // with the counters, within plm_gemm_noalloc's fixed scratch
+// Partial sums of a call's K split: with the counters, within plm_gemm_noalloc's fixed scratch, so that it
+// gives plm_gemm's bits. (W8A8, which has no such form, keeps the same limit. A tail's K split is bounded by
+// the caller's bytes alone.)
+constexpr int64_t kMfmaMaxPartials = 24 << 20;
 
 mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, int64_t limit) {
     const mfma_mode mode = a8 ? kModeA8 : (f == PLM_FP8 ? kModeFp8 : kModeInt4);
