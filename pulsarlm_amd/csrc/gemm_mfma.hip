@@ -27,7 +27,10 @@ struct mfma_config {
 // 36.3 -> 27.5 us, fp8 M = 1000, N = 7168, K = 5120 107 -> 79, W8A8 M = 2048, N = 5120, K = 17408
 // 240 -> 219.
 struct shape_cost {
-    double step[3];  // us per K tile with one, two and three workgroups on a CU (0: they do not fit)
+    // us per K tile with one, two and three workgroups on a CU. 0: LDS or registers hold no more, and a
+    // further one waits (fp8 D has two: 186 VGPRs and twice 57 KiB; with a joint rate for three it was picked at
+    // 15-25 % below its time: fp8 M = 402, N = 33888, K = 2688 118.7 us on D, 99.9 on C).
+    double step[3];
     double fill;     // K tiles
 };
 struct mode_cost {
@@ -40,13 +43,13 @@ struct mode_cost {
 constexpr mode_cost kModeCost[3] = {
     // int4: -, R, W, X, Q, -, H, -, B, C, D, F
     {3.64, 2.09, 0.185, 0.0907,
-     {{}, {{0.7425, 1.0481, 1.4028}, 1.29}, {{2.6043, 0, 0}, 2.58}, {{2.6513, 0, 0}, 2.62}, {{0.6862, 1.0969, 1.7074}, 0.85}, {},
+     {{}, {{0.7425, 1.0481, 1.4028}, 1.29}, {{2.6043, 0, 0}, 2.58}, {{2.6513, 0, 0}, 2.62}, {{0.6862, 1.0969, 0}, 0.85}, {},
       {{1.5961, 0, 0}, 3.18}, {}, {{0.9172, 1.8354, 0}, 2.78}, {{1.0175, 1.3798, 0}, 1.59}, {{1.1135, 1.4712, 0}, 2.47},
       {{1.3813, 2.8355, 0}, 3.20}}},
     // fp8 W8A16: -, R, -, X, -, G, -, A, B, C, D, F
     {6.65, 1.09, 0.241, 0.0725,
      {{}, {{1.0994, 1.2560, 1.5931}, 0}, {}, {{3.0932, 0, 0}, 2.89}, {}, {{1.9275, 0, 0}, 0.96}, {}, {{1.4369, 1.6295, 0}, 1.28},
-      {{1.0004, 2.1533, 0}, 0}, {{1.3506, 1.5386, 2.3011}, 0.09}, {{1.4295, 1.6564, 2.6851}, 0.89}, {{1.7632, 3.5806, 0}, 1.43}}},
+      {{1.0004, 2.1533, 0}, 0}, {{1.3506, 1.5386, 2.0}, 0.09}, {{1.4295, 1.6564, 0}, 0.89}, {{1.7632, 3.5806, 0}, 1.43}}},
     // W8A8 (launch: with the quantizer's): S, R, W, X, -, -, H, A, B, C, D, -
     {8.67, 0.25, 0.373, 0.0672,
      {{{0.7845, 0.9704, 0}, 2.92}, {{0.5235, 0.6673, 0.8485}, 5.97}, {{1.4117, 0, 0}, 3.25}, {{1.6860, 0, 0}, 4.27}, {}, {},
