@@ -109,18 +109,20 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
                 if (partials > kMfmaMaxPartials || c.need > limit) break;
                 cost += mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(tiles * splits);
             }
-            // A tail launch: whole rounds, then the rest as halves or with K split. Each launch brings in its
-            // own share of the tiles, and a tail's steps take longer than a whole call's: 1.15 times for
-            // halves; 1.1 times for a K split, and 4 us and 1.5 us for each tile that the last workgroup
-            // adds up. The pick is then 0.5-0.6 % (K split) and 0.6-0.8 % (halves) slower than the faster side, at
-            // about 340 sizes where a tail can be had and comes near; 2.5-5.5 % without tails. fp8 K 5120, N 34816,
-            // M = 2048 762 -> 676 us, K 17408, N 5120, M = 4096 738 -> 650; W8A8 K 5120, N 34816, M = 2048
-            // 406 -> 391; int4 the same size 664 -> 616.
+            // A tail launch: whole rounds, then the rest as halves or with K split, for the shapes of one workgroup
+            // to a CU (beside others the first workgroups that end make room for the last ones; W8A8 H: 9 of
+            // 10 sizes 5-30 % slower). Each launch brings in its own share of the tiles, and a tail's steps
+            // take longer than a whole call's: 1.15 times for halves; 1.1 times for a K split, and 4 us and 6 us for
+            // each MiB that the last workgroup adds up. The pick is then 0.2-0.8 % slower than the faster side, at
+            // about 550 sizes where a tail can be had and comes near; 0.6-5.5 % without tails. us without and with
+            // it: fp8 K 5120, N 34816, M = 2048 762, 676 (X); K 17408, N 5120, M = 2048 475, 370 (G); K 5120 138, 125;
+            // int4 K 13696, N 3744, M = 2228 259, 230 (H); W8A8 K 16896, N 17440, M = 1007 409, 333 (W).
+            const bool tails = sc.step[1] == 0 && !(mode == kModeA8 && id == kIdH);
             const int64_t rem = tiles % cus;
-            if (id == kIdX && splits == 1 && tiles > cus && rem > 0 && 2 * rem <= cus && ktiles >= 8 && !t.mfma_no_tail &&
+            if (tails && splits == 1 && tiles > cus && rem > 0 && 2 * rem <= cus && ktiles >= 8 && !t.mfma_no_tail &&
                 !t.mfma_unsplit && t.mfma_splits == 0) {
                 const double whole = mc.launch + loop(sc, tiles - rem, static_cast<double>(tps), memory(tiles - rem, sh.bm()));
-                if (mode != kModeFp8 && rem % m_blocks == 0 && !t.mfma_no_halves) {
+                if (id == kIdX && mode != kModeFp8 && rem % m_blocks == 0 && !t.mfma_no_halves) {
                     // (fp8 W8A16, whose tall shape keeps the weights in registers, measured slower with halves.)
                     const double both = whole + 1.15 * loop(mc.shapes[kIdH], cus, static_cast<double>(tps), memory(2 * rem, kTallHalf.bm()));
                     if (both < cost) {
@@ -134,7 +136,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
                     const int64_t partials = rem * tsp * sh.bm() * sh.bs() * kTileN * 4;
                     const double steps = loop(sc, cus, static_cast<double>(ttps), memory(rem, sh.bm()));
                     const double exchange = mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(rem * tsp);
-                    const double both = whole + 1.1 * (steps + exchange) + 4.0 + 1.5 * static_cast<double>(tsp);
+                    const double both = whole + 1.1 * (steps + exchange) + 4.0 + 6.0 * tile_mib * static_cast<double>(tsp);
                     if (tsp >= 2 && rem <= kMaxCounters && kCounterBytes + partials <= limit && both < cost) {
                         cost = both;
                         c.tail_tiles = static_cast<int>(rem);

@@ -12,8 +12,8 @@ from tests._util import mfma_plan
     # Two to three workgroups a CU. The 112-row fp8 tile fits two on a CU, not three: us with it first.
     ("fp8", 402, 33888, 2688, (96, 128)),  # 118.7, 99.9
     ("fp8", 215, 36880, 1408, (64, 128)),  # 42.3, 36.1
-    ("fp8", 684, 13856, 14720, (256, 256)),  # 388.4, 355.6
-    ("fp8", 723, 13472, 5248, (128, 128)),  # 147.6, 136.2
+    ("fp8", 2862, 3712, 9856, (256, 256)),  # 254.2, 240.7
+    ("fp8", 598, 16000, 5632, (128, 128)),  # 159.3, 146.1
     # Three of the 96-row tile do: 128-row tiles first.
     ("fp8", 1572, 10096, 1152, (96, 128)),  # 54.1, 46.9
     ("fp8", 801, 19376, 3328, (96, 128)),  # 139.8, 122.3

@@ -143,3 +143,36 @@ def test_plan_follows_the_workspace(fmt, m, n, k):
             assert_close(y, ref, f"{nbytes} of {full} bytes, call {i}")
             assert torch.equal(seen.setdefault(nbytes, y), y), f"{nbytes} of {full} bytes, call {i}"
     assert any(not torch.equal(y, seen[full]) for y in seen.values())
+
+
+@pytest.mark.parametrize("fmt,shape,m,n,k,splits", [
+    ("fp8", "G", 999, 8296, 1408, 2), ("fp8", "G", 1511, 5480, 2944, 5), ("int4", "H", 487, 16616, 2944, 5),
+    ("int4", "H", 743, 10984, 2176, 4), ("w8a8", "W", 999, 12456, 2176, 4)])
+def test_k_split_tails(fmt, shape, m, n, k, splits, tuning_env):
+    """Whole rounds of a shape and the tiles past them with K split, in a second launch: the last row block and
+    the last strip are ragged and lie in the tail."""
+    tuning_env("PLM_MFMA", shape)
+    plan = mfma_plan(fmt, m, n, k)
+    assert plan["tile"][0] == ROWS[shape] and plan["tail"] > 0 and plan["tail_splits"] == splits and not plan["halves"], plan
+    x = to_dev(x_case(m, k, "bf16", seed=m), torch.bfloat16)
+    if fmt == "w8a8":
+        rng = np.random.default_rng(3)
+        codes, scale = O.fp8_block_quantize(O.bf16_round(rng.standard_normal((n, k)).astype(np.float32) * 0.02), 128, 128)
+        w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), to_dev(scale), 128, 128)
+        ref = O.gemm_w8a8_ref(*O.quantize_per_token_e4m3(to_np(x)), codes, scale, 128, 128, dtype=None)
+        run = lambda: ops.gemm_fp8_w8a8_cuda(x, w, sc, n, 128, 128)
+    else:
+        block_n = 1 if fmt == "int4" else 128
+        if fmt == "int4":
+            packed, s = int4_case(n, k, 128, 1, seed=n)
+            w, sc = ops.repack_int4_marlin_cuda(to_dev(packed), scale_tensor(s.astype(np.float16)), 1, 128)
+            run = lambda: ops.gemm_int4_marlin_cuda(x, w, sc, n, 1, 128)
+        else:
+            codes, s = fp8_case(n, k, 128, 128, seed=n)
+            x = (x * 0.05).contiguous()
+            w, sc = ops.repack_fp8_marlin_cuda(to_dev(codes).view(torch.float8_e4m3fn), scale_tensor(s), 128, 128)
+            run = lambda: ops.gemm_fp8_marlin_cuda(x, w, sc, n, 128, 128)
+        ref = to_np(x.double() @ ops.dequant_marlin_cuda(fmt, w, sc, n, k, block_n, 128, torch.bfloat16).double().t())
+    y = run()
+    assert_close(y, ref, f"{fmt} {shape} m={m}")
+    assert torch.equal(y, run()), "not deterministic"
