@@ -21,8 +21,11 @@ struct mfma_config {
 // share it: two cost less than twice one) with a start of `fill` steps, bounded below by the tile
 // bytes that come through L2; a K split adds the exchange of its partial sums. The constants are
 // a fit to 2600 timings: each shape and split at six layers (K = 2048..12288, N = 2048..14336) and
-// nine row counts from 136 to 3300. Over them the pick is 1.3 % (int4), 1.4 % (fp8) and 3 % (W8A8)
-// slower than the best shape. The rule before it counted whole rounds of K tiles times the tile area
+// nine row counts from 136 to 3300. Over them the pick is 1.3 % (int4) and 1.4 % (fp8) slower than the best
+// shape. W8A8 is a fit to 7480 timings at 263 random sizes (M = 33..6000, N = 960..35200, K = 1024..19200), 1.5 %
+// off the best there and 1.4 % at 87 others; with the constants from the six layers 6.9 and 4.9 %, at
+// worst 1.6 times (a start of six K tiles on the 64-row shape sent short calls to others: M = 236, N = 1568,
+// K = 2944 21.7 -> 15.0 us). The rule before it counted whole rounds of K tiles times the tile area
 // over one rate a shape and had no tile heights of 96 and 112 rows: int4 M = 333, N = 6144, K = 4096
 // 36.3 -> 27.5 us, fp8 M = 1000, N = 7168, K = 5120 107 -> 79, W8A8 M = 2048, N = 5120, K = 17408
 // 240 -> 219.
@@ -36,25 +39,26 @@ struct shape_cost {
 struct mode_cost {
     double launch;      // us
     double reduce;      // us a K split
+    double reduce_pass;  // us more for each further pass of the last workgroup over the splits
     double reduce_mib;  // us per MiB of partial sums
     double memory;      // us per MB of x and weight tiles
     shape_cost shapes[kShapes];  // in shape_id order
 };
 constexpr mode_cost kModeCost[3] = {
     // int4: -, R, W, X, Q, -, H, -, B, C, D, F
-    {3.64, 2.09, 0.185, 0.0907,
+    {3.64, 2.09, 0, 0.185, 0.0907,
      {{}, {{0.7425, 1.0481, 1.4028}, 1.29}, {{2.6043, 0, 0}, 2.58}, {{2.6513, 0, 0}, 2.62}, {{0.6862, 1.0969, 0}, 0.85}, {},
       {{1.5961, 0, 0}, 3.18}, {}, {{0.9172, 1.8354, 0}, 2.78}, {{1.0175, 1.3798, 0}, 1.59}, {{1.1135, 1.4712, 0}, 2.47},
       {{1.3813, 2.8355, 0}, 3.20}}},
     // fp8 W8A16: -, R, -, X, -, G, -, A, B, C, D, F
-    {6.65, 1.09, 0.241, 0.0725,
+    {6.65, 1.09, 0, 0.241, 0.0725,
      {{}, {{1.0994, 1.2560, 1.5931}, 0}, {}, {{3.0932, 0, 0}, 2.89}, {}, {{1.9275, 0, 0}, 0.96}, {}, {{1.4369, 1.6295, 0}, 1.28},
       {{1.0004, 2.1533, 0}, 0}, {{1.3506, 1.5386, 2.0}, 0.09}, {{1.4295, 1.6564, 0}, 0.89}, {{1.7632, 3.5806, 0}, 1.43}}},
-    // W8A8 (launch: with the quantizer's): S, R, W, X, -, -, H, A, B, C, D, -
-    {8.67, 0.25, 0.373, 0.0672,
-     {{{0.7845, 0.9704, 0}, 2.92}, {{0.5235, 0.6673, 0.8485}, 5.97}, {{1.4117, 0, 0}, 3.25}, {{1.6860, 0, 0}, 4.27}, {}, {},
-      {{0.9717, 0, 0}, 5.03}, {{0.7791, 1.0045, 0}, 2.87}, {{0.7998, 1.5840, 0}, 1.80}, {{0.6252, 0.8124, 0}, 3.44},
-      {{0.6875, 0.8929, 0}, 3.56}, {}}}};
+    // W8A8 (without the quantizer's launch): S, R, W, X, -, -, H, A, B, C, D, -
+    {5.25, 2.58, 1.64, 0.200, 0.0018,
+     {{{0.7889, 1.0025, 0}, 3.07}, {{0.5777, 0.7136, 0.9246}, 2.50}, {{1.2907, 0, 0}, 4.77}, {{1.6584, 0, 0}, 5.12}, {}, {},
+      {{1.0419, 0, 0}, 4.78}, {{0.7811, 1.0186, 0}, 3.32}, {{0.7656, 1.5312, 0}, 4.77}, {{0.6406, 0.8521, 0}, 2.10},
+      {{0.7151, 0.9370, 0}, 2.74}, {}}}};
 
 // Partial sums of a call's K split: with the counters, within plm_gemm_noalloc's fixed scratch, so that it
 // gives plm_gemm's bits. (W8A8, which has no such form, keeps the same limit. A tail's K split is bounded by
@@ -94,6 +98,10 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
             const double steps = (tps + sc.fill) * g, x = steps * steps * steps, y = floor * floor * floor;
             return std::cbrt(std::sqrt(x * x + y * y));  // the larger one, rounded where they meet
         };
+        auto exchange = [&](int64_t of, int64_t splits) {  // of `of` tiles' partial sums
+            return mc.reduce + mc.reduce_pass * static_cast<double>(ceil_div(splits, split_batch(sh.mt, sh.ns)) - 1) +
+                   mc.reduce_mib * tile_mib * static_cast<double>(of * splits);
+        };
         for (int64_t want = 1; want <= std::min<int64_t>(8, ktiles); ++want) {
             const int64_t tps = ceil_div(ktiles, want), splits = ceil_div(ktiles, tps);
             if (splits != want || (t.mfma_splits > 0 && splits != std::min<int64_t>(t.mfma_splits, ktiles))) continue;
@@ -107,7 +115,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
                 const int64_t partials = tiles * splits * sh.bm() * sh.bs() * kTileN * 4;
                 c.need = kCounterBytes + partials;
                 if (partials > kMfmaMaxPartials || c.need > limit) break;
-                cost += mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(tiles * splits);
+                cost += exchange(tiles, splits);
             }
             // A tail launch: whole rounds, then the rest as halves or with K split, for the shapes of one workgroup
             // to a CU (beside others the first workgroups that end make room for the last ones; W8A8 H: 9 of
@@ -135,8 +143,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
                     const int64_t ttps = ceil_div(ktiles, std::max<int64_t>(ts, 1)), tsp = ceil_div(ktiles, ttps);
                     const int64_t partials = rem * tsp * sh.bm() * sh.bs() * kTileN * 4;
                     const double steps = loop(sc, cus, static_cast<double>(ttps), memory(rem, sh.bm()));
-                    const double exchange = mc.reduce + mc.reduce_mib * tile_mib * static_cast<double>(rem * tsp);
-                    const double both = whole + 1.1 * (steps + exchange) + 4.0 + 6.0 * tile_mib * static_cast<double>(tsp);
+                    const double both = whole + 1.1 * (steps + exchange(rem, tsp)) + 4.0 + 6.0 * tile_mib * static_cast<double>(tsp);
                     if (tsp >= 2 && rem <= kMaxCounters && kCounterBytes + partials <= limit && both < cost) {
                         cost = both;
                         c.tail_tiles = static_cast<int>(rem);

@@ -73,6 +73,9 @@ struct mfma_args {
 
 namespace {
 
+// K splits whose partial sums the last workgroup of a tile loads at a time.
+constexpr int split_batch(int mt, int ns) { return mt * ns <= 4 ? 8 : (mt * ns <= 8 ? 4 : (mt * ns <= 16 ? 2 : 1)); }
+
 template <bool A8> struct a_traits {
     static constexpr int row_bytes = A8 ? kTileK : kTileK * 2;  // one A row of one K tile
     static constexpr int slots = row_bytes / 16;                 // its 16-byte slots
@@ -622,7 +625,7 @@ __global__ void __launch_bounds__(WM * WN * 64) mfma_kernel(mfma_args a) {
             if (!arrive_last(&a.counters[blockIdx.x], static_cast<uint32_t>(a.splits), &last_flag)) return;
             // Several splits' loads in flight where the registers allow (one at a time, each split
             // costs a memory round trip): SB of them, past the last one out of range.
-            constexpr int SB = MT * NS <= 4 ? 8 : (MT * NS <= 8 ? 4 : (MT * NS <= 16 ? 2 : 1));
+            constexpr int SB = split_batch(MT, NS);
             for (int s0 = 0; s0 < a.splits; s0 += SB) {
                 f32x4_t v[SB][MT][NS];
 #pragma unroll

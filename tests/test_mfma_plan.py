@@ -1,4 +1,4 @@
-"""The MFMA kernel's tile shape, on the CPU (where the library counts 256 CUs), at sizes where the shapes were
+"""The MFMA kernel's tile shape and K split, on the CPU (where the library counts 256 CUs), at sizes where the shapes were
 timed against each other."""
 
 from __future__ import annotations
@@ -21,3 +21,15 @@ from tests._util import mfma_plan
 def test_tile(fmt, m, n, k, tile):
     plan = mfma_plan(fmt, m, n, k)
     assert plan["tile"] == tile and plan["splits"] == 1 and plan["tail"] == 0, plan
+
+
+@pytest.mark.parametrize("m,n,k,tile,splits", [
+    # Short W8A8 calls: us on 96- to 128-row tiles with K in 3 to 6, us here.
+    (236, 1568, 2944, (64, 128), 4),  # 21.7, 15.0
+    (325, 1216, 1664, (64, 128), 4),  # 21.2, 14.1 (K in 3)
+    (705, 1152, 1536, (64, 128), 1),  # 19.6, 14.4
+    (570, 5744, 1664, (64, 128), 1),  # 19.3, 16.7
+])
+def test_w8a8(m, n, k, tile, splits):
+    plan = mfma_plan("w8a8", m, n, k)
+    assert plan["tile"] == tile and plan["splits"] == splits and plan["tail"] == 0, plan

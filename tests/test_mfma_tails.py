@@ -16,7 +16,6 @@ from tests._util import mfma_plan
     ("fp8", 1495, 14416, 5632, False),  # 254, 268
     ("int4", 1206, 27632, 16896, True),  # 1218, 956
     ("int4", 2403, 19968, 1408, False),  # 141, 153
-    ("w8a8", 2365, 20672, 7296, True),  # 481, 413
     ("w8a8", 7687, 4176, 7040, False),  # 281, 305
     ("int4", 2048, 34816, 5120, True),  # 664, 616
     ("w8a8", 2048, 34816, 5120, True),  # 406, 391
@@ -41,6 +40,7 @@ def test_tail(fmt, m, n, k, tail):
     ("int4", 422, 35344, 11776, (128, 256), 5),  # 401 (and 436 with an X tail), 368
     ("w8a8", 1007, 17440, 16896, (256, 192), 2),  # 409, 333
     ("w8a8", 450, 33408, 14464, (256, 192), 2),  # 353, 280
+    ("w8a8", 2365, 20672, 7296, (256, 192), 4),  # 481 (and 417 with an X tail), 406
     ("w8a8", 1212, 6544, 15488, (256, 192), 0),  # 168, 197 (128 x 256 tiles)
     ("w8a8", 412, 17312, 17792, (256, 192), 0),  # 186, 228 (128 x 256 tiles)
 ])
