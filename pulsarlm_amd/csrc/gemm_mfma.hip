@@ -61,9 +61,11 @@ constexpr mode_cost kModeCost[3] = {
       {{0.7151, 0.9370, 0}, 2.74}, {}}}};
 
 // Partial sums of a call's K split: with the counters, within plm_gemm_noalloc's fixed scratch, so that it
-// gives plm_gemm's bits. (W8A8, which has no such form, keeps the same limit. A tail's K split is bounded by
-// the caller's bytes alone.)
+// gives plm_gemm's bits. W8A8, which has no such form, may fill what its calls must bring anyway (K 17536,
+// N 3344, M = 1130: 135 us whole, 99 with K in 2 and 31 MiB of sums). A tail's K split is bounded by the caller's bytes.
 constexpr int64_t kMfmaMaxPartials = 24 << 20;
+
+int64_t mfma_contract_bytes(plm_format f, int64_t m, int64_t n, int64_t k, bool a8);
 
 mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, int64_t limit) {
     const mfma_mode mode = a8 ? kModeA8 : (f == PLM_FP8 ? kModeFp8 : kModeInt4);
@@ -72,6 +74,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
     const int64_t cus = cu_count(), strips = ceil_div(n, kTileN), ktiles = ceil_div(k, kTileK);
     mfma_config best;
     double least = 0;
+    const int64_t most = std::max(kCounterBytes + kMfmaMaxPartials, a8 ? mfma_contract_bytes(f, m, n, k, a8) : 0);
     int forced = -1;  // PLM_MFMA (tuning sweeps)
     for (int id = 0; id < kShapes; ++id)
         if (t.mfma_shape == kShapeLetter[id] && (kModeShapes[mode] >> id & 1)) forced = id;
@@ -114,7 +117,7 @@ mfma_config choose_mfma(plm_format f, int64_t m, int64_t n, int64_t k, bool a8, 
             if (splits > 1) {
                 const int64_t partials = tiles * splits * sh.bm() * sh.bs() * kTileN * 4;
                 c.need = kCounterBytes + partials;
-                if (partials > kMfmaMaxPartials || c.need > limit) break;
+                if (c.need > most || c.need > limit) break;
                 cost += exchange(tiles, splits);
             }
             // A tail launch: whole rounds, then the rest as halves or with K split, for the shapes of one workgroup

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import pytest
 
+from pulsarlm_amd import _lib
 from tests._util import mfma_plan
 
 
@@ -33,3 +34,18 @@ def test_tile(fmt, m, n, k, tile):
 def test_w8a8(m, n, k, tile, splits):
     plan = mfma_plan("w8a8", m, n, k)
     assert plan["tile"] == tile and plan["splits"] == splits and plan["tail"] == 0, plan
+
+
+@pytest.mark.parametrize("m,n,k,tile,splits", [
+    # Sums of more than 24 MiB, which the call must bring anyway: us whole, us here.
+    (1130, 3344, 17536, (128, 128), 2),  # 136, 99
+    (363, 10368, 16384, (128, 128), 2),  # 106, 83
+    (1185, 2704, 15744, (112, 128), 2),  # 103, 82
+])
+def test_w8a8_sums_fill_what_the_call_must_bring(m, n, k, tile, splits, tuning_env):
+    plan = mfma_plan("w8a8", m, n, k)
+    assert plan["tile"] == tile and plan["splits"] == splits and plan["tail"] == 0, plan
+    size = _lib.load().plm_gemm_w8a8_workspace_bytes
+    wanted = size(m, n, k)
+    tuning_env("PLM_MFMA_UNSPLIT", "1")  # no partial sums: the bytes that any plan's call must bring
+    assert size(m, n, k) == wanted
